@@ -141,6 +141,22 @@ struct DirectArgs {
   int32_t g8;  // threads per pixel (power of two >= ceil(M/8))
 };
 
+// Direct 3x3 conv of a narrow layer on padded NHWC fp16 (direct.hip). Work
+// items are 1 output row x one segment of pixels, ordered (n, segment, row)
+// with the row fastest.
+struct DirectRowArgs {
+  const uint16_t* in;  // padded NHWC fp16 [N][Hp][Wp][C]
+  const uint16_t* w;   // direct taps (direct_rows_halfs layout)
+  const float* bias;   // [16 * ceil(M / 16)] fp32, zero padded
+  const uint16_t* skip0;  // padded NHWC fp16 [N][Hp][Wp][M], or null
+  const uint16_t* skip1;  // or null (only with skip0)
+  uint16_t* out;          // padded NHWC fp16 [N][Hp][Wp][M]
+  int32_t N, H, W, Hp, Wp, M;
+  int32_t act;
+  int32_t n_seg, n_items;  // segments per row; N * n_seg * H
+  FastDiv fd_H, fd_seg;
+};
+
 // Elementwise / layout kernels for the ops the conv epilogues do not absorb.
 enum UnaryOp : int32_t { kUnarySigmoid = 0, kUnaryRelu = 1, kUnaryClip = 2 };
 enum BinaryOp : int32_t { kBinaryAdd = 0, kBinaryMul = 1 };

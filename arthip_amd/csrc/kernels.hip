@@ -2827,6 +2827,7 @@ hipError_t launch_winograd(WinoArgs a, hipStream_t s) {
   if (a.in_nchw) return pipe_boundary_eligible(a) ? launch_strip(a, s) : hipErrorInvalidValue;
   if (a.epi.out_kind == kOutNchwF16 && pipe_boundary_eligible(a)) return launch_strip(a, s);
   if (narrow_launch_eligible(a)) return launch_narrow(a, s);
+  if (conv_head_eligible(a)) return launch_conv_head(a, s);
   if (strip_eligible(a)) return launch_strip(a, s);
   const WinoGeom g = winograd_geom(a.C, a.M);
   a.n_ob = g.n_ob;

@@ -42,6 +42,11 @@ hipError_t launch_rowpipe(StripArgs a, int act, int io, hipStream_t s);
 bool rowpipe96_eligible(int C, int M, int nskip, int act, int64_t N, int64_t H, int64_t W,
                         int io);
 hipError_t launch_rowpipe96(StripArgs a, int act, hipStream_t s);
+// Direct convs of narrow layers (direct.hip): whether a conv runs there, and
+// its launch (refused otherwise). conv_head: C = 2 - 4, M = 32, 64 or 96
+// without residual inputs.
+bool conv_head_eligible(const WinoArgs& w);
+hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s);
 hipError_t launch_eltwise(EltArgs a, bool binary, hipStream_t s);
 hipError_t launch_dts(DtsArgs a, hipStream_t s);
 hipError_t launch_input_convert(IoArgs a, hipStream_t s);

@@ -27,8 +27,31 @@ size_t block_u_halfs(int C, int M) {
 
 size_t block_u_offset(int C, int M) { return winograd_u_halfs(C, M) + narrow_packed_halfs(C, M); }
 
+bool direct_head_shape(int C, int M) {
+  return C >= 2 && C <= 4 && (M == 32 || M == 64 || M == 96);
+}
+
+size_t direct_rows_halfs(int C, int M) {
+  return direct_head_shape(C, M) ? static_cast<size_t>(M / 16) * 64 * 16 : 0;
+}
+
+size_t direct_rows_offset(int C, int M) { return block_u_offset(C, M) + block_u_halfs(C, M); }
+
 size_t winograd_packed_halfs(int C, int M) {
-  return winograd_u_halfs(C, M) + narrow_packed_halfs(C, M) + block_u_halfs(C, M);
+  return direct_rows_offset(C, M) + direct_rows_halfs(C, M);
+}
+
+// Direct taps of a narrow layer (layout in pack.h); `out` is zero-filled.
+static void direct_rows_pack(const float* w, int M, int C, uint16_t* out) {
+  const int n_ob = (M + 15) / 16;
+  for (int m = 0; m < M; ++m) {
+    const int b = m % (4 * n_ob) / 4, i = m / (4 * n_ob) * 4 + m % 4;  // A row i of block b
+    for (int dy = 0; dy < 3; ++dy)
+      for (int k = 0; k < 3 * C; ++k) {
+        const float v = w[(static_cast<size_t>(m) * C + k % C) * 9 + dy * 3 + k / C];
+        out[(static_cast<size_t>(b) * 64 + dy * 16 + i) * 16 + k] = f32_to_f16(v);
+      }
+  }
 }
 
 void winograd_pack(const float* w, int M, int C, uint16_t* out) {
@@ -72,6 +95,7 @@ void winograd_pack(const float* w, int M, int C, uint16_t* out) {
       }
     }
   }
+  if (direct_rows_halfs(C, M) != 0) direct_rows_pack(w, M, C, out + direct_rows_offset(C, M));
   for (int m = 0; m < M; ++m) {
     const int ob = m / 16, row = m % 16;
     for (int c = 0; c < C; ++c) {

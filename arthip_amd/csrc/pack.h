@@ -36,7 +36,8 @@ size_t narrow_packed_halfs(int C, int M);
 
 // Halfs in the packed buffer: U' as [n_ob][16 positions][kc][64 lanes][8],
 // followed by the narrow taps when narrow_eligible(C, M), followed for
-// C = M = 64 and C = M = 96 by the row-Winograd filters (block_u_halfs).
+// C = M = 64 and C = M = 96 by the row-Winograd filters (block_u_halfs),
+// followed by the direct taps of a narrow layer (direct_rows_halfs).
 size_t winograd_packed_halfs(int C, int M);
 // The row-Winograd kernels (the fused residual block and the row pipes,
 // C = M = 64 or 96) run F(2,3) along x and sum the three kernel rows in the
@@ -48,6 +49,17 @@ size_t block_u_halfs(int C, int M);
 size_t block_u_offset(int C, int M);
 // Halfs of the U' part alone (offset of the narrow taps).
 size_t winograd_u_halfs(int C, int M);
+// Narrow layers that run as a direct conv (direct.hip). In NHWC the three
+// pixels of a kernel row dy are 3 C contiguous values, value k = dx * C + c.
+// Head shape (C = 2 - 4, M = 32, 64, 96): [M / 16][64 lanes][16], lane
+// (q, i) = q * 16 + i holds values 0 .. 11 of row dy = q (q < 3) of the channel
+// of A row i, the rest zero. A row i of block b is channel
+// 4 n_ob (i / 4) + 4 b + i % 4, so that a lane of the result holds contiguous
+// channels.
+bool direct_head_shape(int C, int M);
+// Halfs of these taps (0 for other shapes) and their offset in the packed buffer.
+size_t direct_rows_halfs(int C, int M);
+size_t direct_rows_offset(int C, int M);
 // w is OIHW [M][C][3][3] fp32 (exact fp16 values from the model).
 void winograd_pack(const float* w, int M, int C, uint16_t* out);
 
