@@ -141,6 +141,19 @@ struct DirectArgs {
   int32_t g8;  // threads per pixel (power of two >= ceil(M/8))
 };
 
+// Contiguous ranges of a launch's work items, one per workgroup slot: slot s
+// takes items [s q + min(s, r), (s + 1) q + min(s + 1, r)), which needs no
+// division on the GPU (a 64-bit one is some 130 instructions).
+struct ItemSplit {
+  int32_t q, r;
+};
+inline ItemSplit make_split(int32_t n_items, int32_t slots) {
+  return ItemSplit{n_items / slots, n_items % slots};
+}
+__host__ __device__ inline int32_t split_begin(ItemSplit s, int32_t slot) {
+  return slot * s.q + (slot < s.r ? slot : s.r);
+}
+
 // Direct 3x3 conv of a narrow layer on padded NHWC fp16 (direct.hip). Work
 // items are 1 output row x one segment of pixels, ordered (n, segment, row)
 // with the row fastest.
@@ -153,7 +166,10 @@ struct DirectRowArgs {
   uint16_t* out;          // padded NHWC fp16 [N][Hp][Wp][M]
   int32_t N, H, W, Hp, Wp, M;
   int32_t act;
+  int32_t nt_out;          // output stores carry the non-temporal hint
   int32_t n_seg, n_items;  // segments per row; N * n_seg * H
+  int32_t seg_w;           // pixels per segment (the last may have fewer)
+  ItemSplit split;
   FastDiv fd_H, fd_seg;
 };
 

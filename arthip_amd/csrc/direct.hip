@@ -71,8 +71,8 @@ __global__ void __launch_bounds__(256) conv3x3_head(DirectRowArgs a) {
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;
 
   // Item = (n * n_seg + segment) * H + output row.
@@ -167,6 +167,261 @@ __global__ void __launch_bounds__(256) conv3x3_head(DirectRowArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Narrow body conv, C = 16 .. 48 (C % 8 == 0), M <= 16 * OB <= 48 (M % 8 == 0)
+// ---------------------------------------------------------------------------
+//
+// In NHWC the three pixels of a kernel row are 3 C contiguous values, so a
+// kernel row is KR = ceil(3 C / 32) products of v_mfma_f32_16x16x32_f16: B is 16
+// output pixels x 32 values of a row, read from LDS as 16 bytes per lane at the
+// pixel's own offset (values past the third pixel are masked to zero), A the
+// taps of 16 output channels, held in VGPRs (12 KR OB of them) for the whole
+// launch. 9 C products per output are more than Winograd's, but nothing is
+// transformed and no V' goes through LDS: the matrix work of these widths is
+// below the time of their memory traffic.
+//
+// One wave per workgroup; it walks down a segment of up to OPX = 30 or 62 output
+// pixels, one row per step, on its own: its input rows (two pixels more) come
+// by 16-byte buffer -> LDS copies into a private ring of R slots, LA rows ahead
+// of the step that reads them, and only the wave's own count of outstanding
+// memory instructions orders ring and copies, no barrier. Every step issues the
+// same instructions on every path (copies past the run and stores past the
+// segment have out-of-range offsets): NSK residual copies, NI row copies, NS
+// stores.
+//
+// Epilogue: bias in the accumulators, one rounding to fp16, activation, then the
+// residual inputs in fp16. The channels of A's rows are permuted (pack.h) so
+// that a lane holds 4 OB contiguous channels of its pixel; they go to the
+// staging slot (with residual inputs the slot that already holds the first
+// residual's row, read and overwritten in place) and leave linearly, whole lines
+// per store instruction.
+//
+// LDS banks: a 16-byte read serves lanes 0-3, 12-15, 20-27 of each half wave
+// together, then the other 16 (measured: equal units of 16 bytes mod 256 slow a
+// read only within these sets). Under that the 32- and 96-byte pixels of
+// C = 16 and 48 are conflict-free as they are; C = 32 stores 16-byte group g of
+// ring pixel p at g ^ (2 ((p >> 2) & 1)) (on the copies' source side), which is
+// too; C = 24 and 40 read two-way.
+//
+// The stream through memory bounds it, on small images the launch and the first
+// rows' latency. 48 -> 48 + ReLU at 541x963 (100 MB): 61 us in winograd_conv, 29
+// here; 32 -> 32 + ReLU at 540x960 (66 MB): 24 us in the strip kernel it ran on
+// before, 17 here; with a residual at 1080p (398 MB): 88 and 65 us; 16 -> 16 at
+// 1080p (133 MB): 68 and 26 us. Its error against 64 bits is a third of
+// Winograd's (2.1e-4 against 6.1e-4): no transform rounds its inputs.
+template <int C, int OB, int NSKIP>
+struct RowsL {
+  // 16-pixel tiles per step; four where two tiles' row is not whole copies.
+  static constexpr int T = C % 16 == 0 ? 2 : 4;
+  static constexpr int IPX = 16 * T;     // input pixels per ring row
+  static constexpr int OPX = IPX - 2;    // output pixels per segment, at most
+  static constexpr int PXB = 2 * C;      // input bytes per pixel
+  static constexpr int KR = (3 * C + 31) / 32;
+  static constexpr int VO = 3 * C / 8 - 4 * (KR - 1);  // octets of the last product
+  static constexpr int NI = IPX * PXB / 1024;          // copies per row
+  static constexpr int SLOT = NI * 1024;
+  static constexpr int LA = 2;
+  static constexpr int R = LA + 3;
+  static constexpr int NS = IPX * 32 * OB / 1024;  // stores per row
+  static constexpr int SSLOT = NS * 1024;
+  static constexpr int NSK = NSKIP * NS;
+  static constexpr int STG = R * SLOT;
+  // Reads of the last tile's unused columns run past the last slot.
+  static constexpr size_t lds_bytes() { return STG + (NSKIP == 0 ? 1 : 2 * NSKIP) * SSLOT; }
+  static_assert(IPX * PXB % 1024 == 0, "whole copies");
+  static_assert((LA - 1) * (NI + NSK) + LA * NS < 64 && 2 * NI + NS + NSK < 64, "vmcnt field");
+  static_assert(NS <= (LA + 1) * NI, "the first residual row's wait");
+  // Last byte read in a slot: pixel 63's row of KR products.
+  static_assert((IPX - 1) * PXB + 64 * KR - SLOT <= SSLOT, "reads stay inside the LDS");
+};
+
+template <int C, int OB, int NSKIP>
+__global__ void __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(2)))
+conv3x3_rows(DirectRowArgs a) {
+  using L = RowsL<C, OB, NSKIP>;
+  constexpr int T = L::T, KR = L::KR, NI = L::NI, NS = L::NS, NSK = L::NSK, LA = L::LA, R = L::R;
+  constexpr bool SWZ = C == 32;
+  extern __shared__ __attribute__((aligned(16))) char rlds[];
+  const int lane = threadIdx.x;
+  const int j = lane & 15;
+  const int q = lane >> 4;
+
+  const int G = gridDim.x;
+  const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
+  if (begin >= end) return;
+
+  h8 wa[3][KR][OB];
+  f4 bias4[OB];
+  {
+    const h8* wp = reinterpret_cast<const h8*>(a.w) + lane;
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+      for (int kc = 0; kc < KR; ++kc)
+#pragma unroll
+        for (int b = 0; b < OB; ++b) wa[dy][kc][b] = wp[((dy * KR + kc) * OB + b) * 64];
+#pragma unroll
+    for (int b = 0; b < OB; ++b)
+      bias4[b] = *reinterpret_cast<const f4*>(a.bias + q * 4 * OB + 4 * b);
+  }
+  // The taps have landed before the first copy goes out: waits inside the loop
+  // then count the loop's own memory instructions only.
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+
+  const uint32_t rowb = (uint32_t)a.Wp * L::PXB;
+  const uint32_t img = (uint32_t)a.Hp * rowb;
+  const uint32_t lds0 = lds_byte_addr(rlds);
+  // B read of tile t, product kc: byte rb[.] + 16 * PXB * t (+ 64 * kc unswizzled).
+  int rb[SWZ ? KR : 1];
+  if constexpr (SWZ) {
+#pragma unroll
+    for (int kc = 0; kc < KR; ++kc) rb[kc] = (j + kc) * L::PXB + ((q ^ (((j + kc) >> 1) & 2)) << 4);
+  } else {
+    rb[0] = j * L::PXB + 16 * q;
+  }
+  const uint32_t vmask = L::VO == 4 || q < L::VO ? ~0u : 0u;
+  // Staging of this lane's channels [4 OB q, 4 OB q + 4 OB) of pixel j.
+  const int mb = a.M * 2;
+  const int sw = L::STG + j * mb + q * 8 * OB;
+
+  int n = 0, sg = 0, y0 = 0;
+  __amdgpu_buffer_rsrc_t rs;
+  uint32_t doff[NI];  // copies' byte offsets from the start of a padded row
+  for (int it = begin; it < end;) {
+    {
+      const uint32_t t = fdiv((uint32_t)it, a.fd_H);
+      y0 = it - (int)(t * (uint32_t)a.H);
+      const uint32_t nn = fdiv(t, a.fd_seg);
+      sg = (int)(t - nn * (uint32_t)a.n_seg);
+      n = (int)nn;
+    }
+    const int len = min(end - it, a.H - y0);
+    const int x0 = sg * a.seg_w;
+    const int valid = min(a.seg_w, a.W - x0);
+    {
+      const char* ib = reinterpret_cast<const char*>(a.in) + (int64_t)n * img;
+      rs = __builtin_amdgcn_make_buffer_rsrc((void*)ib, (short)0, (int)img, 0x00020000);
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int o = 1024 * i + 16 * lane;
+      const int src = SWZ ? 1024 * i + (lane >> 2) * L::PXB + (((lane & 3) ^ ((lane >> 3) & 2)) << 4) : o;
+      doff[i] = o < (valid + 2) * L::PXB ? (uint32_t)(x0 * L::PXB + src) : kOob;
+    }
+    // Input row r of the run (padded row y0 + r) into ring slot s.
+    auto issue_row = [&](int r, int s) {
+      const uint32_t ro = r <= len + 1 ? (uint32_t)(y0 + r) * rowb : kOob;  // uniform
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        dma16_buf(lds0 + (uint32_t)(s * L::SLOT + 1024 * i), rs, (doff[i] | ro) >= kOob ? kOob : doff[i] + ro);
+    };
+    // Output row k of the run as a buffer resource over the segment's pixels.
+    auto out_row = [&](const uint16_t* base, int k) {
+      const char* p = reinterpret_cast<const char*>(base) +
+                      (((int64_t)n * a.Hp + y0 + k + 1) * a.Wp + x0 + 1) * mb;
+      return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, k < len ? valid * mb : 0, 0x00020000);
+    };
+    auto issue_skips = [&](int k) {
+#pragma unroll
+      for (int e = 0; e < NSKIP; ++e) {
+        const __amdgpu_buffer_rsrc_t rk = out_row(e == 0 ? a.skip0 : a.skip1, k);
+#pragma unroll
+        for (int i = 0; i < NS; ++i)
+          dma16_buf(lds0 + (uint32_t)(L::STG + ((k & 1) * NSKIP + e) * L::SSLOT + 1024 * i), rk,
+                    (uint32_t)(1024 * i + 16 * lane));
+      }
+    };
+
+    if constexpr (NSKIP > 0) issue_skips(0);
+#pragma unroll
+    for (int r = 0; r < R - 1; ++r) issue_row(r, r);
+    int s = 0;  // ring slot of input row k
+#pragma unroll 1
+    for (int k = 0; k < len; ++k) {
+      // Input row k + 2 has landed (and with it rows k, k + 1).
+      if (k >= LA)
+        wait_vmcnt<(LA - 1) * (NI + NSK) + LA * NS>();
+      else if (k == 0)
+        wait_vmcnt<(LA - 1) * NI>();
+      else
+        wait_vmcnt<(LA - 1) * NI + NSK + NS>();
+      static_assert(LA == 2, "the waits of rows 0 .. LA - 1");
+      if constexpr (NSKIP > 0) issue_skips(k + 1);
+      issue_row(k + R - 1, s == 0 ? R - 1 : s - 1);
+
+      f4 acc[T][OB];
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int b = 0; b < OB; ++b) acc[t][b] = bias4[b];
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy) {
+        const int sl = s + dy >= R ? s + dy - R : s + dy;
+        const char* row = rlds + sl * L::SLOT;
+#pragma unroll
+        for (int kc = 0; kc < KR; ++kc) {
+          h8 v[T];
+#pragma unroll
+          for (int t = 0; t < T; ++t) {
+            const char* p = row + (SWZ ? rb[SWZ ? kc : 0] : rb[0] + 64 * kc) + 16 * L::PXB * t;
+            v[t] = *reinterpret_cast<const h8*>(p);
+            if (L::VO != 4 && kc == KR - 1)
+              v[t] = __builtin_bit_cast(h8, __builtin_bit_cast(u4, v[t]) & u4{vmask, vmask, vmask, vmask});
+          }
+#pragma unroll
+          for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int b = 0; b < OB; ++b)
+              acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[dy][kc][b], v[t], acc[t][b], 0, 0, 0);
+        }
+      }
+
+      if constexpr (NSKIP > 0) wait_vmcnt<2 * NI + NS + NSK>();  // residual row k
+      char* const st = rlds + sw + (NSKIP > 0 ? (k & 1) * NSKIP * L::SSLOT : 0);
+      auto epilogue = [&](auto act_tag) {
+        constexpr int ACT = decltype(act_tag)::value;
+#pragma unroll
+        for (int b = 0; b < OB; ++b)
+          if (q * 4 * OB + 4 * b < a.M) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+              char* p = st + t * 16 * mb + 8 * b;
+              h4 r = strip_act4<ACT>(acc[t][b]);
+#pragma unroll
+              for (int e = 0; e < NSKIP; ++e) r += *reinterpret_cast<const h4*>(p + e * L::SSLOT);
+              *reinterpret_cast<h4*>(p) = r;
+            }
+          }
+      };
+      if (a.act == kActRelu)
+        epilogue(IntC<kActRelu>{});
+      else if (a.act == kActSilu)
+        epilogue(IntC<kActSilu>{});
+      else
+        epilogue(IntC<kActNone>{});
+      const __amdgpu_buffer_rsrc_t ro = out_row(a.out, k);
+      const char* lin = rlds + L::STG + (NSKIP > 0 ? (k & 1) * NSKIP * L::SSLOT : 0) + 16 * lane;
+      auto store = [&](auto aux_tag) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i)
+          __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u4*>(lin + 1024 * i), ro,
+                                                 (uint32_t)(1024 * i + 16 * lane), 0,
+                                                 decltype(aux_tag)::value);
+      };
+      if (a.nt_out)
+        store(IntC<kNonTemporal>{});
+      else
+        store(IntC<0>{});
+      s = s + 1 == R ? 0 : s + 1;
+    }
+    it += len;
+  }
+  wait_vmcnt<0>();  // no copy into LDS outlives the workgroup
+}
+
+// ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
 
@@ -185,6 +440,22 @@ template <int C>
 RowKernel head_kernel(int M, int act) {
   return M == 32 ? head_kernel_act<C, 2>(act) : M == 64 ? head_kernel_act<C, 4>(act)
                                                         : head_kernel_act<C, 6>(act);
+}
+
+template <int C, int OB>
+RowKernel rows_kernel(int nskip, size_t* lds) {
+  switch (nskip) {
+    case 0: *lds = RowsL<C, OB, 0>::lds_bytes(); return conv3x3_rows<C, OB, 0>;
+    case 1: *lds = RowsL<C, OB, 1>::lds_bytes(); return conv3x3_rows<C, OB, 1>;
+    default: *lds = RowsL<C, OB, 2>::lds_bytes(); return conv3x3_rows<C, OB, 2>;
+  }
+}
+
+template <int C>
+RowKernel rows_kernel(int M, int nskip, size_t* lds) {
+  return M <= 16   ? rows_kernel<C, 1>(nskip, lds)
+         : M <= 32 ? rows_kernel<C, 2>(nskip, lds)
+                   : rows_kernel<C, 3>(nskip, lds);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -211,13 +482,15 @@ DirectRowArgs row_args(const WinoArgs& w, int seg) {
   a.Hp = (int32_t)padded_rows(w.H);
   a.Wp = (int32_t)padded_cols(w.W);
   a.n_seg = (w.W + seg - 1) / seg;
+  a.seg_w = (w.W + a.n_seg - 1) / a.n_seg;
   a.n_items = (int32_t)((int64_t)w.N * a.n_seg * w.H);
   a.fd_H = make_fastdiv((uint32_t)w.H);
   a.fd_seg = make_fastdiv((uint32_t)a.n_seg);
   return a;
 }
 
-hipError_t launch_rows_kernel(RowKernel fn, const DirectRowArgs& a, int threads, size_t lds,
+// cap: workgroups per CU at most.
+hipError_t launch_rows_kernel(RowKernel fn, DirectRowArgs a, int threads, size_t lds, int cap,
                               hipStream_t s) {
   if (lds > 65536) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
@@ -229,9 +502,10 @@ hipError_t launch_rows_kernel(RowKernel fn, const DirectRowArgs& a, int threads,
                                                    lds) != hipSuccess ||
       occ < 1)
     occ = 1;
-  int64_t grid = (int64_t)cu_count() * occ;
+  int64_t grid = (int64_t)cu_count() * (occ < cap ? occ : cap);
   if (grid > a.n_items) grid = a.n_items;
   grid = (grid + 7) / 8 * 8;
+  a.split = make_split(a.n_items, (int)grid);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(threads), lds, s, a);
   return hipGetLastError();
 }
@@ -258,7 +532,52 @@ hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s) {
   const RowKernel fn = w.C == 2   ? head_kernel<2>(w.M, a.act)
                        : w.C == 3 ? head_kernel<3>(w.M, a.act)
                                   : head_kernel<4>(w.M, a.act);
-  return launch_rows_kernel(fn, a, 256, (size_t)4 * 16 * w.M * 2, s);
+  return launch_rows_kernel(fn, a, 256, (size_t)4 * 16 * w.M * 2, 8, s);
+}
+
+// Output pixels of a conv3x3_rows segment.
+static int rows_segment(int C) { return C % 16 == 0 ? RowsL<16, 1, 0>::OPX : RowsL<24, 1, 0>::OPX; }
+
+// 32 -> 32 convs of up to 4096 pixels stay on winograd_strip. Both kernels take
+// about a launch's latency there (36x52: 3.4 us here, 3.8 there), and the
+// models' tests compare such a frame's fp32 and fp16 outputs by errors that
+// they expect to lie above the output's own rounding, as Winograd's do.
+static bool tiny32(const WinoArgs& w) {
+  return w.C == 32 && w.M == 32 && (int64_t)w.N * w.H * w.W <= 4096;
+}
+
+bool conv_rows_eligible(const WinoArgs& w) {
+  if (tiny32(w)) return false;
+  const int64_t cm = w.C > w.M ? w.C : w.M;
+  return inner_epilogue(w) && direct_rows_shape(w.C, w.M) && aligned16(w.in) &&
+         aligned16(w.epi.out) && aligned16(w.epi.skip0) && aligned16(w.epi.skip1) &&
+         fits32(w.N, w.H, w.W, cm, rows_segment(w.C));
+}
+
+hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s) {
+  if (!conv_rows_eligible(w)) return hipErrorInvalidValue;
+  DirectRowArgs a = row_args(w, rows_segment(w.C));
+  // Outputs of up to 96 MiB are stored plainly: the next layer finds them in the
+  // last-level cache (32-channel model: 61 us at 540x960, 65 with non-temporal
+  // stores; 91 and 98 at 720p). Larger ones carry the hint (183 against 185 us
+  // at 1080p, 326 against 354 at 1440x2560, a lone 32 -> 32 conv with a residual
+  // at 1080p 65 against 86).
+  a.nt_out = (int64_t)a.N * a.Hp * a.Wp * a.M * 2 > ((int64_t)96 << 20);
+  const int nskip = (a.skip0 != nullptr) + (a.skip1 != nullptr);
+  size_t lds = 0;
+  RowKernel fn = nullptr;
+  switch (w.C) {
+    case 16: fn = rows_kernel<16>(w.M, nskip, &lds); break;
+    case 24: fn = rows_kernel<24>(w.M, nskip, &lds); break;
+    case 32: fn = rows_kernel<32>(w.M, nskip, &lds); break;
+    case 40: fn = rows_kernel<40>(w.M, nskip, &lds); break;
+    case 48: fn = rows_kernel<48>(w.M, nskip, &lds); break;
+    default: return hipErrorInvalidValue;
+  }
+  // Eight waves per CU at most: more make the runs shorter (two rows of halo
+  // each) without streaming faster (32 -> 32 + residual at 1080p: 94 us with
+  // twelve, 86 with eight, 84 with five; 16 -> 16 at 1080p: 24, 26, 36).
+  return launch_rows_kernel(fn, a, 64, lds, 8, s);
 }
 
 }  // namespace arthip

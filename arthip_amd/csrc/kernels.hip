@@ -2615,8 +2615,9 @@ StripKernel strip_kernel_act(int act, int nskip) {
   }
 }
 
-// winograd_strip covers C == M in {32, 64} with the fast epilogue;
-// winograd_pipe covers C == M = 64 without residual inputs and C == M = 96.
+// C == M in {32, 64, 96} with the fast epilogue: winograd_strip covers 64
+// channels with residual inputs and the 32-channel convs that conv3x3_rows
+// leaves, the row pipes and winograd_pipe the rest.
 bool strip_eligible(const WinoArgs& a) {
   const bool fast_epi = a.epi.out_kind == kOutPadded && a.epi.dts_b < 2 && !a.epi.do_clip &&
                         (a.epi.act == kActNone || a.epi.act == kActRelu ||
@@ -2828,6 +2829,7 @@ hipError_t launch_winograd(WinoArgs a, hipStream_t s) {
   if (a.epi.out_kind == kOutNchwF16 && pipe_boundary_eligible(a)) return launch_strip(a, s);
   if (narrow_launch_eligible(a)) return launch_narrow(a, s);
   if (conv_head_eligible(a)) return launch_conv_head(a, s);
+  if (conv_rows_eligible(a)) return launch_conv_rows(a, s);
   if (strip_eligible(a)) return launch_strip(a, s);
   const WinoGeom g = winograd_geom(a.C, a.M);
   a.n_ob = g.n_ob;

@@ -44,9 +44,12 @@ bool rowpipe96_eligible(int C, int M, int nskip, int act, int64_t N, int64_t H, 
 hipError_t launch_rowpipe96(StripArgs a, int act, hipStream_t s);
 // Direct convs of narrow layers (direct.hip): whether a conv runs there, and
 // its launch (refused otherwise). conv_head: C = 2 - 4, M = 32, 64 or 96
-// without residual inputs.
+// without residual inputs; conv_rows: C = 16 - 48 and M = 8 - 48, multiples of
+// 8, with up to two residual inputs.
 bool conv_head_eligible(const WinoArgs& w);
 hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s);
+bool conv_rows_eligible(const WinoArgs& w);
+hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s);
 hipError_t launch_eltwise(EltArgs a, bool binary, hipStream_t s);
 hipError_t launch_dts(DtsArgs a, hipStream_t s);
 hipError_t launch_input_convert(IoArgs a, hipStream_t s);

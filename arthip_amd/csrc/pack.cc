@@ -31,8 +31,14 @@ bool direct_head_shape(int C, int M) {
   return C >= 2 && C <= 4 && (M == 32 || M == 64 || M == 96);
 }
 
+bool direct_rows_shape(int C, int M) {
+  return C % 8 == 0 && C >= 16 && C <= 48 && M % 8 == 0 && M >= 8 && M <= 48;
+}
+
 size_t direct_rows_halfs(int C, int M) {
-  return direct_head_shape(C, M) ? static_cast<size_t>(M / 16) * 64 * 16 : 0;
+  if (direct_head_shape(C, M)) return static_cast<size_t>(M / 16) * 64 * 16;
+  if (direct_rows_shape(C, M)) return static_cast<size_t>(3 * ((3 * C + 31) / 32)) * ((M + 15) / 16) * 64 * 8;
+  return 0;
 }
 
 size_t direct_rows_offset(int C, int M) { return block_u_offset(C, M) + block_u_halfs(C, M); }
@@ -44,12 +50,17 @@ size_t winograd_packed_halfs(int C, int M) {
 // Direct taps of a narrow layer (layout in pack.h); `out` is zero-filled.
 static void direct_rows_pack(const float* w, int M, int C, uint16_t* out) {
   const int n_ob = (M + 15) / 16;
+  const int kr = (3 * C + 31) / 32;
+  const bool head = direct_head_shape(C, M);
   for (int m = 0; m < M; ++m) {
     const int b = m % (4 * n_ob) / 4, i = m / (4 * n_ob) * 4 + m % 4;  // A row i of block b
     for (int dy = 0; dy < 3; ++dy)
       for (int k = 0; k < 3 * C; ++k) {
         const float v = w[(static_cast<size_t>(m) * C + k % C) * 9 + dy * 3 + k / C];
-        out[(static_cast<size_t>(b) * 64 + dy * 16 + i) * 16 + k] = f32_to_f16(v);
+        const size_t idx =
+            head ? (static_cast<size_t>(b) * 64 + dy * 16 + i) * 16 + k
+                 : (((static_cast<size_t>(dy) * kr + k / 32) * n_ob + b) * 64 + k % 32 / 8 * 16 + i) * 8 + k % 8;
+        out[idx] = f32_to_f16(v);
       }
   }
 }

@@ -56,7 +56,11 @@ size_t winograd_u_halfs(int C, int M);
 // of A row i, the rest zero. A row i of block b is channel
 // 4 n_ob (i / 4) + 4 b + i % 4, so that a lane of the result holds contiguous
 // channels.
+// Body shape (C = 16 - 48, M = 8 - 48, multiples of 8): [3 rows dy][ceil(3 C /
+// 32)][n_ob][64 lanes][8] in MFMA A-operand order, lane (q, i) holding values
+// 32 kc + 8 q .. + 7 of row dy of the channel of A row i, the rest zero.
 bool direct_head_shape(int C, int M);
+bool direct_rows_shape(int C, int M);
 // Halfs of these taps (0 for other shapes) and their offset in the packed buffer.
 size_t direct_rows_halfs(int C, int M);
 size_t direct_rows_offset(int C, int M);

@@ -53,6 +53,49 @@ def test_head_nonfinite(c):
     _nonfinite_stays_local(c, 64, 9, 131)
 
 
+# conv3x3_rows: one wave per segment of up to 62 pixels (four 16-pixel tiles), one
+# output row per step, input rows two steps ahead: runs of one, two and three
+# rows, segment edges, many rows per wave, several runs per wave (many segments,
+# few rows).
+ROWS_SIZES = [(1, 1, 1), (2, 2, 15), (1, 3, 17), (3, 5, 61), (1, 2, 62), (1, 1, 63), (2, 4, 125), (1, 700, 130),
+              (1, 3, 4001), (2, 67, 1921)]
+
+
+def _skips(seed, k, n, m, h, w):
+    rng = np.random.default_rng(seed)
+    return [rng.standard_normal((n, m, h, w)).astype(np.float16) for _ in range(k)]
+
+
+@pytest.mark.parametrize("n,h,w", ROWS_SIZES)
+@pytest.mark.parametrize("c,m,k", [(16, 16, 1), (24, 24, 2), (32, 32, 0), (48, 48, 1)])
+def test_rows(c, m, k, n, h, w):
+    x, wt, b = make_case(60, n, c, m, h, w)
+    sk = _skips(61, k, n, m, h, w)
+    check(run_conv(x, wt, b, 1, sk), oracle_conv(x, wt, b, 1, sk), f"rows c{c}m{m} skip{k} {n}x{h}x{w}")
+
+
+@pytest.mark.parametrize("c", [16, 24, 32, 40, 48])
+@pytest.mark.parametrize("m", [8, 16, 24, 32, 40, 48])
+def test_rows_channels(c, m):
+    k = (c + m) // 8 % 3
+    x, wt, b = make_case(62, 1, c, m, 13, 70)
+    sk = _skips(63, k, 1, m, 13, 70)
+    check(run_conv(x, wt, b, 0, sk), oracle_conv(x, wt, b, 0, sk), f"rows c{c}m{m} skip{k}")
+
+
+@pytest.mark.parametrize("act", [0, 1, 2])
+@pytest.mark.parametrize("k", [0, 1, 2])
+def test_rows_epilogue(act, k):
+    x, wt, b = make_case(64, 1, 48, 48, 19, 66)
+    sk = _skips(65, k, 1, 48, 19, 66)
+    check(run_conv(x, wt, b, act, sk), oracle_conv(x, wt, b, act, sk), f"rows act{act} skip{k}")
+
+
+@pytest.mark.parametrize("c", [16, 24, 32, 40, 48])
+def test_rows_nonfinite(c):
+    _nonfinite_stays_local(c, 16, 9, 131, _skips(66, 1, 1, 16, 9, 131))
+
+
 def _run_offset(x, wt, b, skip, off):
     """run_conv with every activation buffer `off` bytes into its allocation."""
     import torch
@@ -80,8 +123,10 @@ def _run_offset(x, wt, b, skip, off):
     return o[:, 1:h + 1, 1:w + 1].astype(np.float32).transpose(0, 3, 1, 2)
 
 
-@pytest.mark.parametrize("c,m", [(3, 64)])
-def test_unaligned_buffers(c, m):
+@pytest.mark.parametrize("c,m,k", [(3, 64, 0), (32, 32, 1), (48, 24, 1)])
+def test_unaligned_buffers(c, m, k):
     """Buffers on 8 bytes only: accepted, by the general kernel."""
     x, wt, b = make_case(53, 1, c, m, 21, 67)
-    check(_run_offset(x, wt, b, None, 8), oracle_conv(x, wt, b, 1), f"offset c{c}m{m}")
+    sk = _skips(54, k, 1, m, 21, 67)
+    got = _run_offset(x, wt, b, sk[0] if k else None, 8)
+    check(got, oracle_conv(x, wt, b, 1, sk), f"offset c{c}m{m}")
