@@ -86,6 +86,7 @@ struct BlockL {
   static constexpr int RROW = 4 * WPS;            // halfs per transformed row
   static constexpr int RPAIR = 2 * RROW;          // halfs per ring slot (row pair)
   static constexpr int NSLOT = 3;
+  static constexpr int FILL = 5;  // what another strip costs a workgroup, in items
   static constexpr int THREADS = 768;             // 12 waves, three per SIMD
   static constexpr int SBUF = StripStage<2>::SBUF;
   static constexpr int RSLOT = 2 * 32 * C;        // halfs per t ring slot (2 t rows x 32 px)
@@ -209,8 +210,8 @@ winograd_block(BlockArgs a) {
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;  // uniform across the workgroup
 
   const int64_t row_bytes = (int64_t)a.Wp * PX;
@@ -549,6 +550,7 @@ hipError_t launch_block(BlockArgs a, hipStream_t s) {
   int64_t grid = cu_count();  // one workgroup per CU (12 waves, 128 KB of LDS)
   if (grid > items) grid = items;
   grid = (grid + 7) / 8 * 8;
+  a.split = make_split(a.n_items, (int)grid, a.tiles_h, BlockL::FILL);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(BlockL::THREADS), lds, s, a);
   return hipGetLastError();
 }

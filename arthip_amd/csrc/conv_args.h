@@ -70,6 +70,19 @@ struct FastDiv {
   uint32_t d, m, s;
 };
 
+// Contiguous ranges of a launch's work items, one per workgroup slot, in the
+// order of strips of equal length (make_split on the host, split_begin on the
+// GPU). Entering a strip costs a workgroup the fill and drain of its pipeline;
+// with pad > 0 each strip is counted as pad items longer, so that a range which
+// crosses into a new strip gets that many items fewer than one which does not.
+// No 64-bit division on the GPU (some 130 instructions each).
+struct ItemSplit {
+  int32_t q, r;   // slot s starts at padded item s q + floor(s r / slots)
+  int32_t pad;
+  FastDiv strip;  // padded strip length
+  FastDiv slots;
+};
+
 // Winograd F(2x2,3x3) conv with C == M in {32, 64} and the fast epilogue
 // (winograd_strip in kernels.hip). Work items are 1 tile row x 16 tile columns,
 // ordered (n, strip of 16 tile columns, tile row) with the tile row fastest, so
@@ -84,6 +97,7 @@ struct StripArgs {
   int32_t N, H, W, Hp, Wp;
   int32_t tiles_h, tiles_w, n_strips;
   int32_t n_items;  // N * n_strips * tiles_h
+  ItemSplit split;
   FastDiv fd_tiles_h, fd_strips;
 };
 
@@ -108,6 +122,7 @@ struct BlockArgs {
   int32_t cached_out;
   int32_t tiles_h, n_strips;
   int32_t n_items;  // N * n_strips * tiles_h
+  ItemSplit split;
   FastDiv fd_tiles_h, fd_strips;
 };
 
@@ -124,6 +139,7 @@ struct NarrowArgs {
   float clip_lo, clip_hi;
   int32_t dts_b, cout;       // DepthToSpace block (1 = none); Cout = M / b^2
   int32_t n_seg, n_items;    // ceil(W / 64); N * n_seg * H
+  ItemSplit split;
   FastDiv fd_H, fd_seg;
   int64_t img_bytes;         // bytes of one output image (< 2^31)
 };
@@ -140,19 +156,6 @@ struct DirectArgs {
   int32_t Hp, Wp;
   int32_t g8;  // threads per pixel (power of two >= ceil(M/8))
 };
-
-// Contiguous ranges of a launch's work items, one per workgroup slot: slot s
-// takes items [s q + min(s, r), (s + 1) q + min(s + 1, r)), which needs no
-// division on the GPU (a 64-bit one is some 130 instructions).
-struct ItemSplit {
-  int32_t q, r;
-};
-inline ItemSplit make_split(int32_t n_items, int32_t slots) {
-  return ItemSplit{n_items / slots, n_items % slots};
-}
-__host__ __device__ inline int32_t split_begin(ItemSplit s, int32_t slot) {
-  return slot * s.q + (slot < s.r ? slot : s.r);
-}
 
 // Direct 3x3 conv of a narrow layer on padded NHWC fp16 (direct.hip). Work
 // items are 1 output row x one segment of pixels, ordered (n, segment, row)

@@ -491,7 +491,7 @@ DirectRowArgs row_args(const WinoArgs& w, int seg) {
 
 // cap: workgroups per CU at most.
 hipError_t launch_rows_kernel(RowKernel fn, DirectRowArgs a, int threads, size_t lds, int cap,
-                              hipStream_t s) {
+                              int fill, hipStream_t s) {
   if (lds > 65536) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -505,7 +505,7 @@ hipError_t launch_rows_kernel(RowKernel fn, DirectRowArgs a, int threads, size_t
   int64_t grid = (int64_t)cu_count() * (occ < cap ? occ : cap);
   if (grid > a.n_items) grid = a.n_items;
   grid = (grid + 7) / 8 * 8;
-  a.split = make_split(a.n_items, (int)grid);
+  a.split = make_split(a.n_items, (int)grid, a.H, fill);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(threads), lds, s, a);
   return hipGetLastError();
 }
@@ -532,7 +532,7 @@ hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s) {
   const RowKernel fn = w.C == 2   ? head_kernel<2>(w.M, a.act)
                        : w.C == 3 ? head_kernel<3>(w.M, a.act)
                                   : head_kernel<4>(w.M, a.act);
-  return launch_rows_kernel(fn, a, 256, (size_t)4 * 16 * w.M * 2, 8, s);
+  return launch_rows_kernel(fn, a, 256, (size_t)4 * 16 * w.M * 2, 8, 0, s);
 }
 
 // Output pixels of a conv3x3_rows segment.
@@ -577,7 +577,7 @@ hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s) {
   // Eight waves per CU at most: more make the runs shorter (two rows of halo
   // each) without streaming faster (32 -> 32 + residual at 1080p: 94 us with
   // twelve, 86 with eight, 84 with five; 16 -> 16 at 1080p: 24, 26, 36).
-  return launch_rows_kernel(fn, a, 64, lds, 8, s);
+  return launch_rows_kernel(fn, a, 64, lds, 8, 1, s);
 }
 
 }  // namespace arthip

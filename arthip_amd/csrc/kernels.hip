@@ -435,8 +435,8 @@ winograd_strip(StripArgs a) {
   // contiguous eighth of the items.
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;  // uniform across the workgroup
 
   h8 u[16][KC];
@@ -813,8 +813,8 @@ winograd_pipe(StripArgs a) {
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;  // uniform across the workgroup
   const int K = end - begin;
 
@@ -1316,8 +1316,8 @@ conv3x3_narrow(NarrowArgs a) {
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;  // uniform across the workgroup
 
   h8 wb[9][KC];
@@ -1533,8 +1533,8 @@ conv3x3_tail(NarrowArgs a) {
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;  // uniform across the workgroup
 
   h8 wb[3][KC];
@@ -1850,7 +1850,7 @@ __global__ void __launch_bounds__(256) direct_conv_c1(DirectArgs a) {
 constexpr int HEAD_ROWS = 6;
 
 template <int G8, int ACT, bool SKIP, int BIN>
-__global__ void __launch_bounds__(256) direct_conv_c1_walk(DirectArgs a, int n_seg, int n_items,
+__global__ void __launch_bounds__(256) direct_conv_c1_walk(DirectArgs a, int n_seg, ItemSplit split,
                                                            FastDiv fd_seg, FastDiv fd_H) {
   constexpr int SEG = 4 * 256 / G8;
   constexpr int NR = HEAD_ROWS;
@@ -1875,8 +1875,8 @@ __global__ void __launch_bounds__(256) direct_conv_c1_walk(DirectArgs a, int n_s
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)n_items * slot / G);
-  const int end = (int)((int64_t)n_items * (slot + 1) / G);
+  const int begin = split_begin(split, slot);
+  const int end = split_begin(split, slot + 1);
   if (begin >= end) return;
 
   // Item = (n * n_seg + segment) * H + output row.
@@ -2040,7 +2040,7 @@ __global__ void __launch_bounds__(256) direct_conv_c1_walk(DirectArgs a, int n_s
 // products are exact in fp32 and summed in the matrix unit; the epilogue is
 // fast4, as in the other head kernels.
 template <int NB, int ACT, int BIN>
-__global__ void __launch_bounds__(256) direct_conv_c1_mfma(DirectArgs a, int n_seg, int n_items,
+__global__ void __launch_bounds__(256) direct_conv_c1_mfma(DirectArgs a, int n_seg, ItemSplit split,
                                                            FastDiv fd_seg, FastDiv fd_H) {
   static_assert(NB % 2 == 0 && NB <= 6, "16 * NB output channels, NB even");
   constexpr int M = 16 * NB;
@@ -2070,8 +2070,8 @@ __global__ void __launch_bounds__(256) direct_conv_c1_mfma(DirectArgs a, int n_s
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)n_items * slot / G);
-  const int end = (int)((int64_t)n_items * (slot + 1) / G);
+  const int begin = split_begin(split, slot);
+  const int end = split_begin(split, slot + 1);
   if (begin >= end) return;
 
   // Item = (n * n_seg + segment) * H + output row.
@@ -2627,7 +2627,7 @@ bool strip_eligible(const WinoArgs& a) {
 }
 
 template <int KC, int NSKIP, int IO = 0>
-hipError_t launch_pipe(const StripArgs& a, int act, hipStream_t s) {
+hipError_t launch_pipe(StripArgs a, int act, hipStream_t s) {
   StripKernel pf = act == kActRelu   ? winograd_pipe<KC, kActRelu, NSKIP, IO>
                    : act == kActSilu ? winograd_pipe<KC, kActSilu, NSKIP, IO>
                                      : winograd_pipe<KC, kActNone, NSKIP, IO>;
@@ -2650,6 +2650,7 @@ hipError_t launch_pipe(const StripArgs& a, int act, hipStream_t s) {
       }
   }
   grid = (grid + 7) / 8 * 8;
+  a.split = make_split(a.n_items, (int)grid, a.tiles_h, 3);
   hipLaunchKernelGGL(pf, dim3((unsigned)grid), dim3(512), lds, s, a);
   return hipGetLastError();
 }
@@ -2738,6 +2739,7 @@ hipError_t launch_strip(const WinoArgs& w, hipStream_t s) {
   int64_t grid = (int64_t)cu_count() * occ;
   if (grid > items) grid = items;
   grid = (grid + 7) / 8 * 8;
+  a.split = make_split(a.n_items, (int)grid, a.tiles_h, 1);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(threads), lds, s, a);
   return hipGetLastError();
 }
@@ -2763,7 +2765,7 @@ bool narrow_launch_eligible(const WinoArgs& w) {
 }
 
 template <int KC>
-hipError_t launch_narrow_kc(const NarrowArgs& a, bool f32, hipStream_t s) {
+hipError_t launch_narrow_kc(NarrowArgs a, bool f32, hipStream_t s) {
   const bool rows = narrow_row_packed(a.M);
   NarrowKernel fn = rows ? (f32 ? conv3x3_tail<KC, true> : conv3x3_tail<KC, false>)
                          : (f32 ? conv3x3_narrow<KC, true> : conv3x3_narrow<KC, false>);
@@ -2782,6 +2784,7 @@ hipError_t launch_narrow_kc(const NarrowArgs& a, bool f32, hipStream_t s) {
   int64_t grid = (int64_t)cu_count() * occ;
   if (grid > a.n_items) grid = a.n_items;
   grid = (grid + 7) / 8 * 8;
+  a.split = make_split(a.n_items, (int)grid, a.H, 2);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(threads), lds, s, a);
   return hipGetLastError();
 }
@@ -2894,7 +2897,7 @@ hipError_t launch_direct(DirectArgs a, hipStream_t s) {
                           : head_reads_boundary_input(a.N, a.H, a.W, a.M, a.in_kind == 2);
     if (fits) {
       const FastDiv fs = make_fastdiv((uint32_t)n_seg), fh = make_fastdiv((uint32_t)a.H);
-      using HeadKernel = void (*)(DirectArgs, int, int, FastDiv, FastDiv);
+      using HeadKernel = void (*)(DirectArgs, int, ItemSplit, FastDiv, FastDiv);
       const bool sk = a.epi.skip0 != nullptr || a.epi.skip1 != nullptr;
       if (a.in_kind != 0 && sk) return hipErrorInvalidValue;
       const int act = a.epi.act == kActRelu ? 1 : (a.epi.act == kActSilu ? 2 : 0);
@@ -2942,7 +2945,8 @@ hipError_t launch_direct(DirectArgs a, hipStream_t s) {
           if (grid > mitems) grid = mitems;
           grid = (grid + 7) / 8 * 8;
           const FastDiv fms = make_fastdiv((uint32_t)ns);
-          hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), lds, s, a, ns, (int)mitems, fms, fh);
+          hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), lds, s, a, ns,
+                             make_split((int)mitems, (int)grid, a.H, 0), fms, fh);
           return hipGetLastError();
         }
       }
@@ -2959,7 +2963,8 @@ hipError_t launch_direct(DirectArgs a, hipStream_t s) {
       int64_t grid = (int64_t)cu_count() * (occ > 2 ? 2 : occ);
       if (grid > items) grid = items;
       grid = (grid + 7) / 8 * 8;
-      hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, s, a, n_seg, (int)items, fs, fh);
+      hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, s, a, n_seg,
+                         make_split((int)items, (int)grid, a.H, 1), fs, fh);
       return hipGetLastError();
     }
   }

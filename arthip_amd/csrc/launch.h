@@ -18,6 +18,30 @@ int cu_count();
 // Multiply-shift constants for dividing uniform values < 2^31 by d on the GPU.
 FastDiv make_fastdiv(uint32_t d);
 
+// Ranges of n_items work items (strips of strip_len items) over `slots`
+// workgroups (below 2^15). `fill` is what entering another strip costs a
+// workgroup, in items; strips are padded by it unless the longest unpadded range
+// with the strips that it enters is no longer than the longest padded one: where
+// the slots are a multiple of the strips (1080p: 256 and 64) no range enters any.
+inline ItemSplit make_split(int32_t n_items, int32_t slots, int32_t strip_len, int32_t fill) {
+  const int64_t strips = n_items / strip_len;
+  const int64_t padded = n_items + strips * fill;
+  const int64_t longest = (static_cast<int64_t>(n_items) + slots - 1) / slots;
+  const int64_t enters = slots % strips == 0   ? 0
+                         : strips % slots == 0 ? strips / slots - 1
+                                               : (longest + strip_len - 2) / strip_len;
+  const bool pad = padded < static_cast<int64_t>(1) << 31 &&
+                   (padded + slots - 1) / slots < longest + enters * fill;
+  const int32_t total = pad ? static_cast<int32_t>(padded) : n_items;
+  ItemSplit s{};
+  s.pad = pad ? fill : 0;
+  s.q = total / slots;
+  s.r = total % slots;
+  s.strip = make_fastdiv(static_cast<uint32_t>(strip_len + s.pad));
+  s.slots = make_fastdiv(static_cast<uint32_t>(slots));
+  return s;
+}
+
 // Largest channel counts the register-resident Winograd kernel is built for.
 int winograd_max_kc();  // input channels <= 32 * winograd_max_kc()
 int winograd_max_m();   // output channels

@@ -63,6 +63,7 @@ struct RowPipeL {
   static constexpr int PX = 2 * C;       // bytes per pixel
   static constexpr int TILES = 32;       // tiles per item
   static constexpr int OPX = 2 * TILES;  // output pixels per item
+  static constexpr int FILL = 3;  // what another strip costs a workgroup, in items
   static constexpr int THREADS = 768;
   static constexpr int WPS = TILES * 64;  // halfs per position (32 tiles x 64 channels)
   static constexpr int RROW = 4 * WPS;    // halfs per transformed row
@@ -219,8 +220,8 @@ winograd_rowpipe(StripArgs a) {
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;  // uniform across the workgroup
 
   const int64_t row_bytes = (int64_t)a.Wp * PX;
@@ -583,6 +584,7 @@ hipError_t launch_rowpipe(StripArgs a, int act, int io, hipStream_t s) {
       }
   }
   grid = (grid + 7) / 8 * 8;
+  a.split = make_split(a.n_items, (int)grid, a.tiles_h, RowPipeL::FILL);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(RowPipeL::THREADS), lds, s, a);
   return hipGetLastError();
 }

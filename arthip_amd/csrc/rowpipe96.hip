@@ -52,6 +52,7 @@ struct RowPipe96L {
   static constexpr int KC = C / 32;       // 32-channel MFMA chunks
   static constexpr int TILES = 16;        // tiles per item
   static constexpr int OPX = 2 * TILES;   // output pixels per item
+  static constexpr int FILL = 3;  // what another strip costs a workgroup, in items
   static constexpr int THREADS = 1024;
   static constexpr int TROW = 112;             // halfs per tile and position (224 bytes)
   static constexpr int WPS = TILES * TROW;     // halfs per position
@@ -143,8 +144,8 @@ winograd_rowpipe96(StripArgs a) {
 
   const int G = gridDim.x;
   const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
-  const int begin = (int)((int64_t)a.n_items * slot / G);
-  const int end = (int)((int64_t)a.n_items * (slot + 1) / G);
+  const int begin = split_begin(a.split, slot);
+  const int end = split_begin(a.split, slot + 1);
   if (begin >= end) return;  // uniform across the workgroup
 
   const int64_t row_bytes = (int64_t)a.Wp * PX;
@@ -424,6 +425,7 @@ hipError_t launch_rowpipe96(StripArgs a, int act, hipStream_t s) {
   int64_t grid = cu_count();  // one workgroup per CU (16 waves, 158 KB of LDS)
   if (grid > items) grid = items;
   grid = (grid + 7) / 8 * 8;
+  a.split = make_split(a.n_items, (int)grid, a.tiles_h, RowPipe96L::FILL);
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(RowPipe96L::THREADS), lds, s, a);
   return hipGetLastError();
 }

@@ -48,6 +48,14 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t x, FastDiv f) {
   return static_cast<uint32_t>((t + x) >> f.s);
 }
 
+// First item of a slot's range (ItemSplit).
+__device__ __forceinline__ int split_begin(const ItemSplit& s, int slot) {
+  const int v = slot * s.q + (int)fdiv((uint32_t)(slot * s.r), s.slots);
+  const int strip = (int)fdiv((uint32_t)v, s.strip);
+  const int len = (int)s.strip.d - s.pad;
+  return strip * len + max(v - strip * (int)s.strip.d - s.pad, 0);
+}
+
 // V' of one input task (4 channels x one tile) into the V' buffer; same
 // transform and scaling as store_v, with the patch rows split in two halves.
 // The patch is held as half2 pairs (element 2*(4*row + col) + e, channel pair
