@@ -64,8 +64,11 @@ namespace arthip {
 //
 // Per run (one strip, output tile rows j0 .. j0+len-1; input row pair Q_i =
 // padded rows 2(j0+i)-1, 2(j0+i); t tile row i covers t rows 2(j0+i)-1 and
-// 2(j0+i), i = 0 .. len), after a prologue that transforms Q_0 into V1 slot
-// 0 and a barrier, phase k (k = 0 .. len+4) ends with the workgroup barrier:
+// 2(j0+i), i = 0 .. len), after a prologue that transforms Q_0 and Q_1 into V1
+// slots 0 and 1 and a barrier, phase k (k = 1 .. len+4) ends with the workgroup
+// barrier (Q_1 in a phase of its own, requested after Q_0's transform, cost
+// every run a load's latency and a barrier: R8F64 at 64x96 70.3 -> 67.8 us, at
+// 333x517 221 -> 215 us, the shipped architecture at 480x853 737 -> 728 us):
 //   conv1 waves:     fold t_{k-1} from V1 slots (k-1)%3, k%3 into ring slot
 //                    (k-1)&1 (1 <= k <= len+1)
 //   conv2 waves:     fold output row k-4 from V2 slots (k-1)%3, k%3 (rows of
@@ -173,14 +176,12 @@ __device__ __forceinline__ void block_fold(const h8 (&u)[3][4][2], const _Float1
   y11 = __builtin_elementwise_fma(X1, m2, c1);
 }
 
-// Phases k = 0 .. len + 4 of one run, six per iteration so that k % 6, and
+// Phases k = 1 .. len + 4 of one run, six per iteration so that k % 6, and
 // with it the t ring and staging parity and the three row-pair slots, is a
 // compile-time constant (every LDS offset an immediate): ph(k6_tag, k).
 template <class F>
 __device__ __forceinline__ void block_phases(int len, F&& ph) {
-  for (int k = 0;;) {
-    ph(IntC<0>{}, k);
-    if (++k > len + 4) break;
+  for (int k = 1;;) {
     ph(IntC<1>{}, k);
     if (++k > len + 4) break;
     ph(IntC<2>{}, k);
@@ -190,6 +191,8 @@ __device__ __forceinline__ void block_phases(int len, F&& ph) {
     ph(IntC<4>{}, k);
     if (++k > len + 4) break;
     ph(IntC<5>{}, k);
+    if (++k > len + 4) break;
+    ph(IntC<0>{}, k);
     if (++k > len + 4) break;
   }
 }
@@ -300,7 +303,7 @@ winograd_block(BlockArgs a) {
         const int tc0 = L::OPX * s - 1 + 2 * tcol;
         cm0 = (tc0 >= 0 && tc0 < a.W) ? ~0u : 0u;
         cm1 = (tc0 + 1 < a.W) ? ~0u : 0u;
-        lds_sync();  // the prologue's transform of Q_0
+        lds_sync();  // the prologue's transforms
         block_phases(len, [&](auto pt, int k) { phase(pt, k, len); });
         it += len;
       }
@@ -479,12 +482,15 @@ winograd_block(BlockArgs a) {
       run_pix = ((int64_t)n * a.Hp + 2 * j0 + 1) * a.Wp + L::OPX * s + 1;
       lane_off = (sx < L::OPX && L::OPX * s + sx < a.W) ? s_lane : kOob;
     }
-    // Prologue: Q_0 (padded rows 2 j0 - 1, 2 j0) into V1 slot 0, then the
-    // rows of Q_1 for phase 0. Slot 0 is free: the last fold of an earlier
-    // run read it at least three barriers ago.
+    // Prologue: Q_0 (padded rows 2 j0 - 1, 2 j0) into V1 slot 0 and Q_1 into
+    // slot 1, both requested at once, then the rows of Q_2 for phase 1. The
+    // slots are free: the last fold of an earlier run read them at least three
+    // barriers ago.
     load2(X, 2 * j0 - 1);
+    load2(T, 2 * j0 + 1);
     row_pair_transform(vw1, X);
-    load2(X, 2 * j0 + 1);
+    load2(X, 2 * j0 + 3);
+    row_pair_transform(vw1 + RPAIR, T);
     lds_sync();  // every role: the prologue's barrier
     block_phases(len, [&](auto pt, int k) { phase(pt, k, len); });
     it += len;

@@ -33,8 +33,8 @@ namespace arthip {
 //     into a 3-slot ring of transformed row pairs (4 positions x 16 tiles x 96
 //     channels per row, 224-byte tile rows) and load the rows of the pair
 //     after it.
-// Phase k (k = 0 .. len+2 of a run, after a prologue that transforms Q_0 into
-// slot 0; Q_i = padded rows 2 (j0 + i), + 1; item i reads Q_i and Q_{i+1})
+// Phase k (k = 1 .. len+2 of a run, after a prologue that transforms Q_0 and Q_1
+// into slots 0 and 1; Q_i = padded rows 2 (j0 + i), + 1; item i reads Q_i and Q_{i+1})
 // ends with the workgroup barrier:
 //   group 1: fold item k-1 from slots (k-1)%3, k%3 and write its partials
 //            P, Q (fp32) to partial buffer (k-1)&1   (1 <= k <= len)
@@ -107,13 +107,11 @@ __device__ __forceinline__ void rp96_transform(_Float16* vw, const h8 (&x)[8]) {
   }
 }
 
-// Phases k = 0 .. len + 2 of a run, six per iteration so that k % 6 (the ring
+// Phases k = 1 .. len + 2 of a run, six per iteration so that k % 6 (the ring
 // slots and the buffer parities) is a compile-time constant.
 template <class F>
 __device__ __forceinline__ void rp96_phases(int len, F&& ph) {
-  for (int k = 0;;) {
-    ph(IntC<0>{}, k);
-    if (++k > len + 2) break;
+  for (int k = 1;;) {
     ph(IntC<1>{}, k);
     if (++k > len + 2) break;
     ph(IntC<2>{}, k);
@@ -123,6 +121,8 @@ __device__ __forceinline__ void rp96_phases(int len, F&& ph) {
     ph(IntC<4>{}, k);
     if (++k > len + 2) break;
     ph(IntC<5>{}, k);
+    if (++k > len + 2) break;
+    ph(IntC<0>{}, k);
     if (++k > len + 2) break;
   }
 }
@@ -376,12 +376,16 @@ winograd_rowpipe96(StripArgs a) {
                        ? (uint32_t)(st_r[e] * rb32 + st_x[e] * PX + st_g[e] * 16)
                        : kOob;
     run_pix = ((int64_t)n * a.Hp + 2 * j0 + 1) * a.Wp + L::OPX * s + 1;
-    // Prologue: Q_0 into slot 0, then the rows of Q_1 for phase 0. Slot 0 is
-    // free: an earlier run's last fold read it at least two barriers ago.
+    // Prologue: Q_0 and Q_1 into slots 0 and 1, then the rows of Q_2 for
+    // phase 1. The slots are free: an earlier run's last fold read them at
+    // least two barriers ago.
     if (has_task) {
+      h8 X1[8];
       load8(X8, 2 * j0);
+      load8(X1, 2 * j0 + 2);
       rp96_transform(vw, X8);
-      load8(X8, 2 * j0 + 2);
+      load8(X8, 2 * j0 + 4);
+      rp96_transform(vw + RPAIR, X1);
     }
     lds_sync();
     rp96_phases(len, [&](auto pt, int k) { phase(pt, k, len); });
