@@ -176,6 +176,15 @@ struct DirectRowArgs {
   FastDiv fd_H, fd_seg;
 };
 
+// A 1 -> 32 head conv on the boundary input and the 32 -> 32 conv that reads it
+// (conv3x3_head_pair): r is the second conv's, with r.in the boundary input
+// [N][1][H][W].
+struct HeadPairArgs {
+  DirectRowArgs r;
+  const uint16_t* w1;  // the head's packed taps (direct_pack)
+  const float* bias1;  // [32] fp32
+};
+
 // Elementwise / layout kernels for the ops the conv epilogues do not absorb.
 enum UnaryOp : int32_t { kUnarySigmoid = 0, kUnaryRelu = 1, kUnaryClip = 2 };
 enum BinaryOp : int32_t { kBinaryAdd = 0, kBinaryMul = 1 };

@@ -9,6 +9,7 @@
 #include "conv_args.h"
 #include "launch.h"
 #include "pack.h"
+#include "plan_rules.h"
 #include "wino_dev.h"
 
 namespace arthip {
@@ -234,6 +235,41 @@ struct RowsL {
   static_assert((IPX - 1) * PXB + 64 * KR - SLOT <= SSLOT, "reads stay inside the LDS");
 };
 
+// Three input rows (ring slots at row[0..2]) times the taps, onto acc: B of tile t,
+// product kc of a row at byte rb[.] + 16 * PXB * t (+ 64 * kc unswizzled).
+template <class L, int OB, int NRB>
+__device__ __forceinline__ void rows_fold(const h8 (&wa)[3][L::KR][OB], const char* const (&row)[3],
+                                          const int (&rb)[NRB], uint32_t vmask, f4 (&acc)[L::T][OB]) {
+  constexpr int T = L::T, KR = L::KR;
+#pragma unroll
+  for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+    for (int kc = 0; kc < KR; ++kc) {
+      h8 v[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const char* p = row[dy] + (NRB > 1 ? rb[kc % NRB] : rb[0] + 64 * kc) + 16 * L::PXB * t;
+        v[t] = *reinterpret_cast<const h8*>(p);
+        if (L::VO != 4 && kc == KR - 1)
+          v[t] = __builtin_bit_cast(h8, __builtin_bit_cast(u4, v[t]) & u4{vmask, vmask, vmask, vmask});
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int b = 0; b < OB; ++b)
+          acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[dy][kc][b], v[t], acc[t][b], 0, 0, 0);
+    }
+}
+
+// One staged output row leaves linearly: NS whole-kilobyte stores from lin.
+template <int NS, int AUX>
+__device__ __forceinline__ void rows_store(const char* lin, __amdgpu_buffer_rsrc_t ro, int lane) {
+#pragma unroll
+  for (int i = 0; i < NS; ++i)
+    __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u4*>(lin + 1024 * i), ro,
+                                           (uint32_t)(1024 * i + 16 * lane), 0, AUX);
+}
+
 template <int C, int OB, int NSKIP>
 __global__ void __launch_bounds__(64)
     __attribute__((amdgpu_waves_per_eu(2)))
@@ -356,27 +392,11 @@ conv3x3_rows(DirectRowArgs a) {
       for (int t = 0; t < T; ++t)
 #pragma unroll
         for (int b = 0; b < OB; ++b) acc[t][b] = bias4[b];
+      const char* row[3];
 #pragma unroll
-      for (int dy = 0; dy < 3; ++dy) {
-        const int sl = s + dy >= R ? s + dy - R : s + dy;
-        const char* row = rlds + sl * L::SLOT;
-#pragma unroll
-        for (int kc = 0; kc < KR; ++kc) {
-          h8 v[T];
-#pragma unroll
-          for (int t = 0; t < T; ++t) {
-            const char* p = row + (SWZ ? rb[SWZ ? kc : 0] : rb[0] + 64 * kc) + 16 * L::PXB * t;
-            v[t] = *reinterpret_cast<const h8*>(p);
-            if (L::VO != 4 && kc == KR - 1)
-              v[t] = __builtin_bit_cast(h8, __builtin_bit_cast(u4, v[t]) & u4{vmask, vmask, vmask, vmask});
-          }
-#pragma unroll
-          for (int t = 0; t < T; ++t)
-#pragma unroll
-            for (int b = 0; b < OB; ++b)
-              acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[dy][kc][b], v[t], acc[t][b], 0, 0, 0);
-        }
-      }
+      for (int dy = 0; dy < 3; ++dy)
+        row[dy] = rlds + (s + dy >= R ? s + dy - R : s + dy) * L::SLOT;
+      rows_fold<L, OB>(wa, row, rb, vmask, acc);
 
       if constexpr (NSKIP > 0) wait_vmcnt<2 * NI + NS + NSK>();  // residual row k
       char* const st = rlds + sw + (NSKIP > 0 ? (k & 1) * NSKIP * L::SSLOT : 0);
@@ -401,24 +421,215 @@ conv3x3_rows(DirectRowArgs a) {
         epilogue(IntC<kActSilu>{});
       else
         epilogue(IntC<kActNone>{});
-      const __amdgpu_buffer_rsrc_t ro = out_row(a.out, k);
       const char* lin = rlds + L::STG + (NSKIP > 0 ? (k & 1) * NSKIP * L::SSLOT : 0) + 16 * lane;
-      auto store = [&](auto aux_tag) {
-#pragma unroll
-        for (int i = 0; i < NS; ++i)
-          __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u4*>(lin + 1024 * i), ro,
-                                                 (uint32_t)(1024 * i + 16 * lane), 0,
-                                                 decltype(aux_tag)::value);
-      };
       if (a.nt_out)
-        store(IntC<kNonTemporal>{});
+        rows_store<NS, kNonTemporal>(lin, out_row(a.out, k), lane);
       else
-        store(IntC<0>{});
+        rows_store<NS, 0>(lin, out_row(a.out, k), lane);
       s = s + 1 == R ? 0 : s + 1;
     }
     it += len;
   }
   wait_vmcnt<0>();  // no copy into LDS outlives the workgroup
+}
+
+// ---------------------------------------------------------------------------
+// Head pair: 1 -> 32 head conv on the boundary input, then a 32 -> 32 conv
+// ---------------------------------------------------------------------------
+//
+// conv3x3_rows whose ring rows are not copied from memory but computed: the head
+// conv of one row (direct_conv_c1_mfma's product, channel order and epilogue,
+// so the same bits as the two convs apart) goes straight into the ring, and its
+// output tensor never exists. Step k computes head row k + 3 while it folds rows
+// k .. k + 2; the input of the row after that is requested a step ahead. Head
+// pixels outside the image are zero: the second conv's padding.
+// The output's write stream and the launch bound it. At 540x960: 11 us for the
+// head and 17 for the conv apart, 18 here; the 32-channel model's frame 62.7 -> 54.7
+// us, at 2x1080x1920 390 -> 301.
+struct HeadPairL : RowsL<32, 2, 0> {
+  static constexpr int R = 4;
+  static constexpr int STG = R * SLOT;
+  static constexpr size_t lds_bytes() { return STG + SSLOT; }
+};
+
+// AUX: the output stores' cache policy (a branch between two kinds of stores
+// would make the compiler's wait counts assume none).
+template <int ACT1, int BIN, int AUX>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+conv3x3_head_pair(HeadPairArgs a) {
+  using L = HeadPairL;
+  constexpr int T = L::T, KR = L::KR, NS = L::NS, R = L::R, OB = 2, NB = 2;
+  constexpr int EB = BIN == 2 ? 4 : 2;  // bytes per input element
+  extern __shared__ __attribute__((aligned(16))) char rlds[];
+  const int lane = threadIdx.x;
+  const int j = lane & 15;
+  const int q = lane >> 4;
+
+  const int G = gridDim.x;
+  const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+  const int begin = split_begin(a.r.split, slot);
+  const int end = split_begin(a.r.split, slot + 1);
+  if (begin >= end) return;
+
+  h8 wa[3][KR][OB];
+  f4 bias4[OB];
+  h4 wh[NB];      // the head's taps, as in direct_conv_c1_mfma
+  f4 hbias[NB];
+  {
+    const h8* wp = reinterpret_cast<const h8*>(a.r.w) + lane;
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+      for (int kc = 0; kc < KR; ++kc)
+#pragma unroll
+        for (int b = 0; b < OB; ++b) wa[dy][kc][b] = wp[((dy * KR + kc) * OB + b) * 64];
+#pragma unroll
+    for (int b = 0; b < OB; ++b) {
+      bias4[b] = *reinterpret_cast<const f4*>(a.r.bias + q * 4 * OB + 4 * b);
+      hbias[b] = *reinterpret_cast<const f4*>(a.bias1 + q * 4 * NB + 4 * b);
+      const int ch = (j >> 2) * 4 * NB + 4 * b + (j & 3);  // A row j of block b
+      const _Float16* tp = reinterpret_cast<const _Float16*>(a.w1) + ch * 10 + 3 * (q < 3 ? q : 0);
+      wh[b] = q < 3 ? h4{tp[0], tp[1], tp[2], (_Float16)0.0f} : h4{0, 0, 0, 0};
+    }
+  }
+  const int H = a.r.H, W = a.r.W;
+  int rb[KR];
+#pragma unroll
+  for (int kc = 0; kc < KR; ++kc) rb[kc] = (j + kc) * L::PXB + ((q ^ (((j + kc) >> 1) & 2)) << 4);
+  const int hw = j * L::PXB + ((q ^ ((j >> 1) & 2)) << 4);  // head pixel j, octet q
+  constexpr int M = 32;
+  const int sw = L::STG + j * M * 2 + q * 8 * OB;
+
+  int n = 0, y0 = 0;
+  const uint32_t img = (uint32_t)H * (uint32_t)W * EB;
+  for (int it = begin; it < end;) {
+    int sg;
+    {
+      const uint32_t t = fdiv((uint32_t)it, a.r.fd_H);
+      y0 = it - (int)(t * (uint32_t)H);
+      const uint32_t nn = fdiv(t, a.r.fd_seg);
+      sg = (int)(t - nn * (uint32_t)a.r.n_seg);
+      n = (int)nn;
+    }
+    const int len = min(end - it, H - y0);
+    const int x0 = sg * a.r.seg_w;
+    const int valid = min(a.r.seg_w, W - x0);
+    const char* ib = reinterpret_cast<const char*>(a.r.in) + (int64_t)n * img;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)ib, (short)0, (int)img, 0x00020000);
+    // Ring pixel p = 16 t + j is image column x0 - 1 + p; its taps the columns
+    // x0 - 2 + p .. x0 + p, as byte offsets in a row (kOob outside the image).
+    uint32_t coff[T][3];
+    uint32_t cmask[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int x = x0 - 1 + 16 * t + j;
+      cmask[t] = x >= 0 && x < W ? ~0u : 0u;
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx) {
+        const int c = x - 1 + dx;
+        coff[t][dx] = c >= 0 && c < W ? (uint32_t)c * EB : kOob;
+      }
+    }
+    // Input of head row r of the run (image row y0 + r - 1): rows y0 + r - 2 + q.
+    // Held as loaded, one value per register: head_row packs them behind an empty
+    // asm statement, else the compiler packs them right after the request and so
+    // waits there, a load's latency per step.
+    uint32_t v[T][3];
+    auto load_row = [&](int r, uint32_t (&v)[T][3]) {
+      const int hr = y0 + r - 2 + q;
+      const uint32_t ro = q < 3 && hr >= 0 && hr < H ? (uint32_t)hr * (uint32_t)W * EB : kOob;
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          const uint32_t o = (coff[t][dx] | ro) >= kOob ? kOob : coff[t][dx] + ro;
+          if constexpr (BIN == 2)
+            v[t][dx] = __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0);
+          else
+            v[t][dx] = __builtin_amdgcn_raw_buffer_load_b16(rs, o, 0, 0);
+        }
+    };
+    auto head_row = [&](int r, int s, uint32_t (&v)[T][3]) {
+      const int y = y0 + r - 1;
+      const uint32_t rmask = y >= 0 && y < H ? ~0u : 0u;  // uniform
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        h4 bv = {0, 0, 0, 0};
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          uint32_t w = v[t][dx];
+          asm volatile("" : "+v"(w));
+          bv[dx] = BIN == 2 ? (_Float16)__builtin_bit_cast(float, w)
+                            : __builtin_bit_cast(_Float16, (uint16_t)w);
+        }
+        const f4 z = {0, 0, 0, 0};
+        const h4 zh = {0, 0, 0, 0};
+        h4 o[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const f4 d = __builtin_amdgcn_mfma_f32_16x16x16f16(wh[b], bv, z, 0, 0, 0) + hbias[b];
+          o[b] = strip_act4<ACT1>(d) + zh;  // (+ 0 as fast4 adds absent residuals)
+        }
+        const u4 m = {rmask & cmask[t], rmask & cmask[t], rmask & cmask[t], rmask & cmask[t]};
+        *reinterpret_cast<u4*>(rlds + s * L::SLOT + hw + 16 * L::PXB * t) =
+            __builtin_bit_cast(u4, __builtin_shufflevector(o[0], o[1], 0, 1, 2, 3, 4, 5, 6, 7)) & m;
+      }
+    };
+    {
+      uint32_t p0[T][3], p1[T][3], p2[T][3];
+      load_row(0, p0);
+      load_row(1, p1);
+      load_row(2, p2);
+      load_row(3, v);
+      head_row(0, 0, p0);
+      head_row(1, 1, p1);
+      head_row(2, 2, p2);
+      // Dropped stores: the loop is entered with the memory instructions of its
+      // back edge (a row's loads, then NS stores), so that its waits for the
+      // loads leave the last step's stores in flight.
+      rows_store<NS, AUX>(rlds + L::STG + 16 * lane,
+                          __builtin_amdgcn_make_buffer_rsrc((void*)a.r.out, (short)0, 0, 0x00020000), lane);
+    }
+    int s = 0;  // ring slot of head row k
+#pragma unroll 1
+    for (int k = 0; k < len; ++k) {
+      const char* row[3];
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy) row[dy] = rlds + ((s + dy) & (R - 1)) * L::SLOT;
+      if (k + 1 < len) {  // uniform
+        head_row(k + 3, (s + 3) & (R - 1), v);
+        load_row(k + 4, v);
+      }
+      f4 acc[T][OB];
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int b = 0; b < OB; ++b) acc[t][b] = bias4[b];
+      rows_fold<L, OB>(wa, row, rb, ~0u, acc);
+      auto epilogue = [&](auto act_tag) {
+        constexpr int ACT = decltype(act_tag)::value;
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          const h4 r0 = strip_act4<ACT>(acc[t][0]), r1 = strip_act4<ACT>(acc[t][1]);
+          *reinterpret_cast<h8*>(rlds + sw + t * 16 * M * 2) =
+              __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+      };
+      if (a.r.act == kActRelu)
+        epilogue(IntC<kActRelu>{});
+      else if (a.r.act == kActSilu)
+        epilogue(IntC<kActSilu>{});
+      else
+        epilogue(IntC<kActNone>{});
+      const char* p = reinterpret_cast<const char*>(a.r.out) +
+                      (((int64_t)n * a.r.Hp + y0 + k + 1) * a.r.Wp + x0 + 1) * (M * 2);
+      rows_store<NS, AUX>(rlds + L::STG + 16 * lane,
+                          __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, valid * M * 2, 0x00020000), lane);
+      s = (s + 1) & (R - 1);
+    }
+    it += len;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -489,9 +700,9 @@ DirectRowArgs row_args(const WinoArgs& w, int seg) {
   return a;
 }
 
-// cap: workgroups per CU at most.
-hipError_t launch_rows_kernel(RowKernel fn, DirectRowArgs a, int threads, size_t lds, int cap,
-                              int fill, hipStream_t s) {
+// Grid of a launch (at most `cap` workgroups per CU) and its ranges in a.split.
+template <class Args>
+hipError_t rows_grid(void (*fn)(Args), DirectRowArgs& a, int threads, size_t lds, int cap, int fill, unsigned* blocks) {
   if (lds > 65536) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -506,8 +717,17 @@ hipError_t launch_rows_kernel(RowKernel fn, DirectRowArgs a, int threads, size_t
   if (grid > a.n_items) grid = a.n_items;
   grid = (grid + 7) / 8 * 8;
   a.split = make_split(a.n_items, (int)grid, a.H, fill);
-  hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(threads), lds, s, a);
-  return hipGetLastError();
+  *blocks = (unsigned)grid;
+  return hipSuccess;
+}
+
+// Outputs of up to 96 MiB are stored plainly: the next layer finds them in the
+// last-level cache (32-channel model: 61 us at 540x960, 65 with non-temporal
+// stores; 91 and 98 at 720p). Larger ones carry the hint (183 against 185 us at
+// 1080p, 326 against 354 at 1440x2560, a lone 32 -> 32 conv with a residual at
+// 1080p 65 against 86).
+bool nt_stores(const DirectRowArgs& a) {
+  return (int64_t)a.N * a.Hp * a.Wp * a.M * 2 > ((int64_t)96 << 20);
 }
 
 // Padded NHWC fp16 on both sides, no Clip, no DepthToSpace.
@@ -528,11 +748,16 @@ bool conv_head_eligible(const WinoArgs& w) {
 
 hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s) {
   if (!conv_head_eligible(w)) return hipErrorInvalidValue;
-  const DirectRowArgs a = row_args(w, 64);
+  DirectRowArgs a = row_args(w, 64);
   const RowKernel fn = w.C == 2   ? head_kernel<2>(w.M, a.act)
                        : w.C == 3 ? head_kernel<3>(w.M, a.act)
                                   : head_kernel<4>(w.M, a.act);
-  return launch_rows_kernel(fn, a, 256, (size_t)4 * 16 * w.M * 2, 8, 0, s);
+  const size_t lds = (size_t)4 * 16 * w.M * 2;
+  unsigned blocks = 0;
+  const hipError_t e = rows_grid(fn, a, 256, lds, 8, 0, &blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(blocks), dim3(256), lds, s, a);
+  return hipGetLastError();
 }
 
 // Output pixels of a conv3x3_rows segment.
@@ -542,12 +767,10 @@ static int rows_segment(int C) { return C % 16 == 0 ? RowsL<16, 1, 0>::OPX : Row
 // about a launch's latency there (36x52: 3.4 us here, 3.8 there), and the
 // models' tests compare such a frame's fp32 and fp16 outputs by errors that
 // they expect to lie above the output's own rounding, as Winograd's do.
-static bool tiny32(const WinoArgs& w) {
-  return w.C == 32 && w.M == 32 && (int64_t)w.N * w.H * w.W <= 4096;
-}
+static bool tiny32(int64_t N, int64_t H, int64_t W) { return N * H * W <= 4096; }
 
 bool conv_rows_eligible(const WinoArgs& w) {
-  if (tiny32(w)) return false;
+  if (w.C == 32 && w.M == 32 && tiny32(w.N, w.H, w.W)) return false;
   const int64_t cm = w.C > w.M ? w.C : w.M;
   return inner_epilogue(w) && direct_rows_shape(w.C, w.M) && aligned16(w.in) &&
          aligned16(w.epi.out) && aligned16(w.epi.skip0) && aligned16(w.epi.skip1) &&
@@ -557,12 +780,7 @@ bool conv_rows_eligible(const WinoArgs& w) {
 hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s) {
   if (!conv_rows_eligible(w)) return hipErrorInvalidValue;
   DirectRowArgs a = row_args(w, rows_segment(w.C));
-  // Outputs of up to 96 MiB are stored plainly: the next layer finds them in the
-  // last-level cache (32-channel model: 61 us at 540x960, 65 with non-temporal
-  // stores; 91 and 98 at 720p). Larger ones carry the hint (183 against 185 us
-  // at 1080p, 326 against 354 at 1440x2560, a lone 32 -> 32 conv with a residual
-  // at 1080p 65 against 86).
-  a.nt_out = (int64_t)a.N * a.Hp * a.Wp * a.M * 2 > ((int64_t)96 << 20);
+  a.nt_out = nt_stores(a);
   const int nskip = (a.skip0 != nullptr) + (a.skip1 != nullptr);
   size_t lds = 0;
   RowKernel fn = nullptr;
@@ -577,7 +795,45 @@ hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s) {
   // Eight waves per CU at most: more make the runs shorter (two rows of halo
   // each) without streaming faster (32 -> 32 + residual at 1080p: 94 us with
   // twelve, 86 with eight, 84 with five; 16 -> 16 at 1080p: 24, 26, 36).
-  return launch_rows_kernel(fn, a, 64, lds, 8, 1, s);
+  unsigned blocks = 0;
+  const hipError_t e = rows_grid(fn, a, 64, lds, 8, 1, &blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(blocks), dim3(64), lds, s, a);
+  return hipGetLastError();
+}
+
+// The conv alone would run conv3x3_rows, and the head direct_conv_c1_mfma on the
+// boundary input: the pair gives the same bits as the two.
+bool head_pair_eligible(int64_t N, int64_t H, int64_t W, bool fp32) {
+  return !tiny32(N, H, W) && fits32(N, H, W, 32, HeadPairL::OPX) && head_reads_boundary_input(N, H, W, 32, fp32);
+}
+
+hipError_t launch_head_pair(const DirectArgs& head, const WinoArgs& conv, hipStream_t s) {
+  if (!head_pair_eligible(head.N, head.H, head.W, head.in_kind == 2) || head.in_kind == 0 || head.M != 32 ||
+      conv.C != 32 || conv.M != 32 || !inner_epilogue(conv) || conv.epi.skip0 != nullptr ||
+      conv.epi.skip1 != nullptr || !aligned16(conv.epi.out))
+    return hipErrorInvalidValue;
+  HeadPairArgs a{};
+  a.r = row_args(conv, HeadPairL::OPX);
+  a.r.in = static_cast<const uint16_t*>(head.in);
+  a.r.nt_out = nt_stores(a.r);
+  a.w1 = head.w;
+  a.bias1 = head.epi.bias;
+  using Fn = void (*)(HeadPairArgs);
+  auto pick = [&](auto bin_tag, auto aux_tag) -> Fn {
+    constexpr int BIN = decltype(bin_tag)::value, AUX = decltype(aux_tag)::value;
+    return head.epi.act == kActRelu   ? conv3x3_head_pair<kActRelu, BIN, AUX>
+           : head.epi.act == kActSilu ? conv3x3_head_pair<kActSilu, BIN, AUX>
+                                      : conv3x3_head_pair<kActNone, BIN, AUX>;
+  };
+  const bool f32 = head.in_kind == 2;
+  const Fn fn = a.r.nt_out ? (f32 ? pick(IntC<2>{}, IntC<kNonTemporal>{}) : pick(IntC<1>{}, IntC<kNonTemporal>{}))
+                           : (f32 ? pick(IntC<2>{}, IntC<0>{}) : pick(IntC<1>{}, IntC<0>{}));
+  unsigned blocks = 0;
+  const hipError_t e = rows_grid(fn, a.r, 64, HeadPairL::lds_bytes(), 8, 2, &blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(blocks), dim3(64), HeadPairL::lds_bytes(), s, a);
+  return hipGetLastError();
 }
 
 }  // namespace arthip

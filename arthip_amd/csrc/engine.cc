@@ -639,8 +639,44 @@ bool Engine::EnsurePlan(Plan& p, const int64_t in[4], std::string& error, void* 
     const Shape si = shapes.at(a.in0);
     return block_eligible(64, 64, a.act, kActNone, si.n, si.h, si.w);
   };
+  // The head conv and the 32 -> 32 conv after it, when that is its only reader:
+  // the head's output then never exists (conv3x3_head_pair).
+  auto pair_at = [&](int i) -> bool {
+    if ((debug_ & kDebugUnfused) || i + 1 >= nops || i != fused_in_op) return false;
+    const Op& a = ops[i];
+    const Op& b = ops[i + 1];
+    if (b.kind != OpKind::Conv || b.in0 != a.out || !b.skips.empty() || b.clip || b.dts_b >= 1) return false;
+    if (a.out == graph_.output_name || readers(a.out) != 1) return false;
+    if (direct_out && i + 1 == final_op) return false;
+    int64_t c1, m1, c2, m2;
+    conv_cm(a, c1, m1);
+    conv_cm(b, c2, m2);
+    return c1 == 1 && m1 == 32 && c2 == 32 && m2 == 32 &&
+           head_pair_eligible(sin.n, sin.h, sin.w, graph_.input_fp32);
+  };
   for (int i = 0; i < nops; ++i) {
     const Op& op = ops[i];
+    if (pair_at(i)) {
+      const Op& op2 = ops[i + 1];
+      if (!alloc(op2.out, shapes.at(op2.out), i)) return fail();
+      Step st;
+      st.kind = StepKind::HeadPair;
+      st.op = i;
+      st.op2 = i + 1;
+      st.in = kBoundaryIn;
+      st.in_kind = graph_.input_fp32 ? 2 : 1;
+      st.out = tbuf.at(op2.out);
+      st.N = (int32_t)sin.n; st.H = (int32_t)sin.h; st.W = (int32_t)sin.w; st.C = 1; st.M = 32;
+      st.wbuf = op_wbuf_.at(i);
+      st.bbuf = op_bbuf_.at(i);
+      st.wbuf2 = op_wbuf_.at(i + 1);
+      st.bbuf2 = op_bbuf_.at(i + 1);
+      st.epi.act = op.act;
+      st.act2 = op2.act;
+      p.steps.push_back(st);
+      ++i;
+      continue;
+    }
     if (block_at(i)) {
       const Op& op2 = ops[i + 1];
       const Shape si = shapes.at(op.in0);
@@ -758,6 +794,7 @@ bool Engine::EnsurePlan(Plan& p, const int64_t in[4], std::string& error, void* 
   auto hbm_bound = [](const Step& n) {
     switch (n.kind) {
       case StepKind::ConvBlock: return false;
+      case StepKind::HeadPair: return false;  // reads the boundary input
       case StepKind::ConvWinograd:
       case StepKind::ConvDirect:
         return n.epi.out_kind != kOutPadded || n.skip[0] != kNoBuffer;
@@ -953,6 +990,24 @@ bool Engine::Enqueue(const Plan& p, const void* in_dev, void* out_dev, hipStream
         e = launch_block(a, s);
         break;
       }
+      case StepKind::HeadPair: {
+        DirectArgs h{};
+        h.in = ptr(st.in);
+        h.in_kind = st.in_kind;
+        h.w = static_cast<const uint16_t*>(wbufs_[st.wbuf].ptr);
+        h.epi.bias = static_cast<const float*>(wbufs_[st.bbuf].ptr);
+        h.epi.act = st.epi.act;
+        h.N = st.N; h.H = st.H; h.W = st.W; h.M = 32;
+        WinoArgs c{};
+        c.u = static_cast<const uint16_t*>(wbufs_[st.wbuf2].ptr);
+        c.epi.bias = static_cast<const float*>(wbufs_[st.bbuf2].ptr);
+        c.epi.out = ptr(st.out);
+        c.epi.act = st.act2;
+        c.epi.out_kind = kOutPadded;
+        c.N = st.N; c.H = st.H; c.W = st.W; c.C = 32; c.M = 32;
+        e = launch_head_pair(h, c, s);
+        break;
+      }
       case StepKind::Eltwise: {
         EltArgs a{};
         a.a = static_cast<const uint16_t*>(ptr(st.in));
@@ -1077,6 +1132,9 @@ std::string Engine::StepName(const Step& st) const {
       for (int k = 0; k < 2; ++k)
         if (st.skip[k] != kNoBuffer) os << " +skip";
       if (st.cached_out) os << " +cached_out";
+      break;
+    case StepKind::HeadPair:
+      os << "head_pair C1 M32" << acts[st.epi.act] << ", C32 M32" << acts[st.act2];
       break;
     case StepKind::Eltwise: os << "eltwise op" << st.elt_op << (st.binary ? " binary" : ""); break;
     case StepKind::DepthToSpace: os << "depth_to_space b" << st.dts_b; break;

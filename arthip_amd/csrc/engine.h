@@ -53,6 +53,7 @@ enum class StepKind {
   ConvWinograd,
   ConvDirect,
   ConvBlock,  // two 64 -> 64 convs fused (winograd_block): op, op2
+  HeadPair,   // a 1 -> 32 head conv and the 32 -> 32 conv after it: op, op2
   Eltwise,
   DepthToSpace,
   OutputConvert
@@ -67,11 +68,12 @@ constexpr int kNoBuffer = -1;
 struct Step {
   StepKind kind = StepKind::ConvWinograd;
   int op = -1;   // index into Graph::ops (-1 for IO steps)
-  int op2 = -1;  // ConvBlock: the second conv
+  int op2 = -1;  // ConvBlock, HeadPair: the second conv
   int in = kNoBuffer, in2 = kNoBuffer, out = kNoBuffer;
   int skip[2] = {kNoBuffer, kNoBuffer};
   int wbuf = kNoBuffer, bbuf = kNoBuffer;  // packed weights / padded bias (weight cache)
-  int wbuf2 = kNoBuffer, bbuf2 = kNoBuffer;  // ConvBlock: the second conv's
+  int wbuf2 = kNoBuffer, bbuf2 = kNoBuffer;  // the second conv's
+  int32_t act2 = kActNone;  // HeadPair: the second conv's activation
   // Geometry of the step's input (NHWC) and channel counts.
   int32_t N = 0, H = 0, W = 0, C = 0, M = 0;
   Epilogue epi{};  // conv epilogue (pointers resolved per run)

@@ -74,6 +74,10 @@ bool conv_head_eligible(const WinoArgs& w);
 hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s);
 bool conv_rows_eligible(const WinoArgs& w);
 hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s);
+// A 1 -> 32 head conv on the NCHW boundary input (fp32: its type) and the
+// 32 -> 32 conv (no residual input) that alone reads it, in one launch.
+bool head_pair_eligible(int64_t N, int64_t H, int64_t W, bool fp32);
+hipError_t launch_head_pair(const DirectArgs& head, const WinoArgs& conv, hipStream_t s);
 hipError_t launch_eltwise(EltArgs a, bool binary, hipStream_t s);
 hipError_t launch_dts(DtsArgs a, hipStream_t s);
 hipError_t launch_input_convert(IoArgs a, hipStream_t s);

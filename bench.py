@@ -406,6 +406,14 @@ def launch_work(spec, steps, px: int):
             # The fused block runs F(2,3) along x, the kernel rows direct: 6 of
             # the 9 products per output and channel pair.
             out.append({"bytes": b, "flops_direct": fd, "flops_wino": fd * 6 / 9, "convs": 2})
+        elif name.startswith("head_pair"):
+            # A head conv and the conv after it, the tensor between them on chip.
+            (c1, m1), _ = convs[ci]
+            (c2, m2), _ = convs[ci + 1]
+            ci += 2
+            b = 2.0 * px * (c1 + m2) + 18.0 * (c1 * m1 + c2 * m2)
+            fd = 2.0 * 9 * px * (c1 * m1 + c2 * m2)
+            out.append({"bytes": b, "flops_direct": fd, "flops_wino": fd, "convs": 2})
         elif name.startswith(("winograd_conv", "direct_conv")):
             (c, m), nsk = convs[ci]
             ci += 1
@@ -415,7 +423,8 @@ def launch_work(spec, steps, px: int):
             # lone 64 -> 64 conv without residual inputs, a 96 -> 96 conv with
             # at most one. Other convs F(2x2,3x3) (16/36).
             rows = (c == m == 64 and nsk == 0) or (c == m == 96 and nsk <= 1)
-            fw = fd if c == 1 else fd * 6 / 9 if rows else fd * 16 / 36
+            direct = c == 1 or 16 <= c <= 48  # direct.hip at the body widths
+            fw = fd if direct else fd * 6 / 9 if rows else fd * 16 / 36
             out.append({"bytes": b, "flops_direct": fd, "flops_wino": fw, "convs": 1})
         else:
             out.append(None)

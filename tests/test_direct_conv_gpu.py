@@ -8,7 +8,8 @@ import ctypes
 import numpy as np
 import pytest
 
-from arthip_amd import _lib
+from arthip_amd import _lib, models
+from arthip_amd.engine import Engine
 from tests.test_conv_kernel_gpu import (check, make_case, oracle_conv, pack, run_conv, to_padded)
 
 pytestmark = pytest.mark.gpu
@@ -94,6 +95,24 @@ def test_rows_epilogue(act, k):
 @pytest.mark.parametrize("c", [16, 24, 32, 40, 48])
 def test_rows_nonfinite(c):
     _nonfinite_stays_local(c, 16, 9, 131, _skips(66, 1, 1, 16, 9, 131))
+
+
+# conv3x3_head_pair (the 32-channel model's head and first conv in one launch)
+# gives the two kernels' bits: its own step against every conv launched alone, on
+# frames above the 4096 pixels from which both run (one segment, many segments,
+# a single row, run boundaries), fp16 and fp32 boundary input.
+@pytest.mark.parametrize("n,h,w", [(1, 69, 61), (2, 33, 125), (1, 1, 4500), (1, 4500, 1), (1, 271, 480)])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_head_pair(n, h, w, fp32):
+    spec = models.c4f32(seed=3)
+    x = models.synthetic_input((n, 1, h, w), seed=5)
+    x = x.astype(np.float32) if fp32 else x
+    model = models.widen_to_fp32(spec) if fp32 else spec
+    with Engine(0) as e, Engine(0) as alone:
+        alone.set_debug(Engine.DEBUG_UNFUSED)
+        got, want = e.build(model).run(x), alone.build(model).run(x)
+        assert "3 launches" in e.describe() and "4 launches" in alone.describe()
+    np.testing.assert_array_equal(got, want)
 
 
 def _run_offset(x, wt, b, skip, off):
