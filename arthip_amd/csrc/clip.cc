@@ -6,6 +6,7 @@
 #include <cstring>
 #include <exception>
 
+#include "host_copy.h"
 #include "launch.h"
 #include "onnx.h"
 
@@ -134,6 +135,7 @@ struct ClipModel::Io {
   void* out_host = nullptr;
   size_t raw_host_cap = 0, raw_dev_cap = 0, in_cap = 0, out_cap = 0, out_int_cap = 0,
          out_host_cap = 0;
+  ChunkedDownload download;
   // Upload landed / kernels done / download done.
   hipEvent_t up = nullptr, comp = nullptr, done = nullptr;
 
@@ -410,9 +412,14 @@ bool ClipModel::RunSlot(Slot& s, Io& io, const VideoFormat& fmt, int in_c, int w
   const size_t obps = out_fp32_ ? 4 : 2;
   const size_t orow = static_cast<size_t>(out_w) * obps;
   const size_t dl_bytes = orow * out_h * n_out;
+  const bool small_out = dl_bytes <= kKernelCopyBytes;
   const bool direct_in = src_kind == in_kind;  // samples already in the boundary type
   for (int c = 0; c < n_out; ++c)
     if (dst_stride[c] < static_cast<ptrdiff_t>(orow)) return fail("destination stride shorter than a row");
+
+  std::vector<HostRows> planes;  // the destination
+  for (int c = 0; c < n_out; ++c)
+    planes.push_back(HostRows{static_cast<uint8_t*>(dst[c]), dst_stride[c], orow, out_h});
 
   hipError_t e = hipSetDevice(device_);
   if (e != hipSuccess) return hip_fail("hipSetDevice", e);
@@ -489,8 +496,13 @@ bool ClipModel::RunSlot(Slot& s, Io& io, const VideoFormat& fmt, int in_c, int w
         !grow_dev(io.out_dev, io.out_cap, out_bytes, aerr) ||
         (int_out && !grow_dev(io.out_int_dev, io.out_int_cap, dl_bytes, aerr)))
       return fail(aerr);
+    // Small transfers are kernels on the engine's own stream, without the copy
+    // streams and their events.
     void* upload_dst = direct_in ? io.in_dev : io.raw_dev;
-    if ((e = hipMemcpyAsync(upload_dst, io.raw_host, raw_bytes, hipMemcpyHostToDevice, s.up)) != hipSuccess ||
+    if (raw_bytes <= kKernelCopyBytes) {
+      if ((e = launch_copy(upload_dst, io.raw_host, raw_bytes, s.stream)) != hipSuccess)
+        return drain(hip_fail("HIP input upload", e));
+    } else if ((e = hipMemcpyAsync(upload_dst, io.raw_host, raw_bytes, hipMemcpyHostToDevice, s.up)) != hipSuccess ||
         (e = hipEventRecord(io.up, s.up)) != hipSuccess ||
         (e = hipStreamWaitEvent(s.stream, io.up, 0)) != hipSuccess)
       return drain(hip_fail("HIP input upload", e));
@@ -510,11 +522,16 @@ bool ClipModel::RunSlot(Slot& s, Io& io, const VideoFormat& fmt, int in_c, int w
       if ((e = launch_plane_convert(pa, s.stream)) != hipSuccess) return drain(hip_fail("plane_convert", e));
       dl_src = io.out_int_dev;
     }
-    if ((e = hipEventRecord(io.comp, s.stream)) != hipSuccess ||
-        (e = hipStreamWaitEvent(s.down, io.comp, 0)) != hipSuccess ||
-        (e = hipMemcpyAsync(io.out_host, dl_src, dl_bytes, hipMemcpyDeviceToHost, s.down)) != hipSuccess)
+    if (small_out) {
+      if ((e = launch_copy(io.out_host, dl_src, dl_bytes, s.stream)) != hipSuccess)
+        return drain(hip_fail("HIP output download", e));
+    } else if ((e = hipEventRecord(io.comp, s.stream)) != hipSuccess ||
+               (e = hipStreamWaitEvent(s.down, io.comp, 0)) != hipSuccess ||
+               (e = io.download.Enqueue(device_, s.down, io.out_host, dl_src, dl_bytes)) != hipSuccess) {
       return drain(hip_fail("HIP output download", e));
-    if ((e = hipEventRecord(io.done, s.down)) != hipSuccess) return drain(hip_fail("HIP event record", e));
+    }
+    const hipStream_t dl_stream = small_out ? s.stream : s.down;
+    if ((e = hipEventRecord(io.done, dl_stream)) != hipSuccess) return drain(hip_fail("HIP event record", e));
     if (prof) {
       if ((e = hipEventSynchronize(io.done)) != hipSuccess) return drain(hip_fail("HIP event synchronize", e));
       std::vector<Engine::StepProfile> steps;
@@ -526,7 +543,7 @@ bool ClipModel::RunSlot(Slot& s, Io& io, const VideoFormat& fmt, int in_c, int w
         hipEvent_t end = nullptr;
         float xfer = 0.0f;
         if (hipEventCreate(&end) == hipSuccess) {
-          if (hipEventRecord(end, s.down) == hipSuccess && hipEventSynchronize(end) == hipSuccess)
+          if (hipEventRecord(end, dl_stream) == hipSuccess && hipEventSynchronize(end) == hipSuccess)
             hipEventElapsedTime(&xfer, s.ev_run, end);
           hipEventDestroy(end);
         }
@@ -539,21 +556,18 @@ bool ClipModel::RunSlot(Slot& s, Io& io, const VideoFormat& fmt, int in_c, int w
       }
     }
   }
-  // Outside the engine lock: wait for this frame's download, copy it out.
-  if ((e = hipEventSynchronize(io.done)) != hipSuccess) return hip_fail("HIP output download", e);
-
-  // Host: rows out of pinned staging into the destination planes.
-  const uint8_t* ost = static_cast<const uint8_t*>(io.out_host);
-  for (int c = 0; c < n_out; ++c) {
-    const uint8_t* from = ost + static_cast<size_t>(c) * orow * out_h;
-    uint8_t* base = static_cast<uint8_t*>(dst[c]);
-    if (dst_stride[c] == static_cast<ptrdiff_t>(orow)) {
-      std::memcpy(base, from, orow * out_h);
-    } else {
-      for (int y = 0; y < out_h; ++y)
-        std::memcpy(base + static_cast<ptrdiff_t>(y) * dst_stride[c], from + static_cast<size_t>(y) * orow, orow);
-    }
+  // Outside the engine lock: this frame's download, copied out as it arrives
+  // (rows out of pinned staging into the destination planes).
+  if (!small_out) {
+    e = io.download.CopyOut(planes);
+    if (e == hipSuccess) e = hipEventSynchronize(io.done);
+    return e == hipSuccess ? true : hip_fail("HIP output download", e);
   }
+  if ((e = hipEventSynchronize(io.done)) != hipSuccess) return hip_fail("HIP output download", e);
+  const uint8_t* ost = static_cast<const uint8_t*>(io.out_host);
+  for (const HostRows& p : planes)
+    for (int y = 0; y < p.rows; ++y, ost += p.row)
+      std::memcpy(p.base + static_cast<ptrdiff_t>(y) * p.stride, ost, p.row);
   return true;
 }
 

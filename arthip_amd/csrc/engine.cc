@@ -1205,25 +1205,37 @@ bool Engine::Run(const void* in_host, const int64_t in[4], void* out_host, size_
     }
   }
   std::memcpy(in_pinned_, in_host, in_bytes);
-  if ((e = hipMemcpyAsync(in_stage_dev_, in_pinned_, in_bytes, hipMemcpyHostToDevice,
-                          stream_)) != hipSuccess) {
+  e = in_bytes <= kKernelCopyBytes
+          ? launch_copy(in_stage_dev_, in_pinned_, in_bytes, stream_)
+          : hipMemcpyAsync(in_stage_dev_, in_pinned_, in_bytes, hipMemcpyHostToDevice, stream_);
+  if (e != hipSuccess) {
     error = HipErr("HIP input upload", e);
     return false;
   }
   rl.Uploaded();
   if (!Enqueue(plan_, in_stage_dev_, out_stage_dev_, stream_, error)) return false;
   rl.Launched();
-  if ((e = hipMemcpyAsync(out_pinned_, out_stage_dev_, out_bytes, hipMemcpyDeviceToHost,
-                          stream_)) != hipSuccess) {
+  const bool small = out_bytes <= kKernelCopyBytes;
+  e = small ? launch_copy(out_pinned_, out_stage_dev_, out_bytes, stream_)
+            : download_.Enqueue(device_, stream_, out_pinned_, out_stage_dev_, out_bytes);
+  if (e != hipSuccess) {
     error = HipErr("HIP output download", e);
     return false;
+  }
+  if (!small) {
+    // Copied out as it arrives; the synchronize below then only reports errors.
+    e = download_.CopyOut({HostRows{static_cast<uint8_t*>(out_host), static_cast<ptrdiff_t>(out_bytes), out_bytes, 1}});
+    if (e != hipSuccess) {
+      error = HipErr("HIP output download", e);
+      return false;
+    }
   }
   if ((e = hipStreamSynchronize(stream_)) != hipSuccess) {
     error = HipErr("HIP stream synchronize", e);
     return false;
   }
   rl.Back();
-  std::memcpy(out_host, out_pinned_, out_bytes);
+  if (small) std::memcpy(out_host, out_pinned_, out_bytes);
   return rl.Done(out_host);
 }
 

@@ -20,6 +20,7 @@
 
 #include "conv_args.h"
 #include "graph.h"
+#include "host_copy.h"
 
 namespace arthip {
 
@@ -219,6 +220,7 @@ class Engine {
   void* out_stage_dev_ = nullptr;
   void* in_pinned_ = nullptr;
   void* out_pinned_ = nullptr;
+  ChunkedDownload download_;
 
   // Profiling: event pairs (step index, start, stop) not yet read.
   bool profiling_ = false;

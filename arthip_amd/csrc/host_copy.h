@@ -1,0 +1,55 @@
+// Device-to-host download of a frame through pinned staging, copied out to the
+// caller's rows as it arrives.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <vector>
+
+namespace arthip {
+
+// Transfers up to this size go by a copy kernel on the launch stream between
+// pinned and device memory: a copy engine's start and the waits between its
+// stream and the kernels cost more than the bytes (R8F64 at 64x96 host to host
+// 114 -> 110 us, a 270x480 frame through the filter 306 -> 288 us).
+constexpr size_t kKernelCopyBytes = static_cast<size_t>(1) << 20;
+
+// `rows` rows of `row` bytes, `stride` bytes apart, of the caller's memory.
+struct HostRows {
+  uint8_t* base;
+  ptrdiff_t stride;
+  size_t row;
+  int rows;
+};
+
+// One download in flight. Enqueue sends it in chunks with an event after each;
+// CopyOut waits for the chunks in order and copies each out while the next ones
+// travel. The copy out of memory that the GPU has just written runs at about
+// half the link's rate on one thread, and the first write to a fresh
+// destination page faults, so larger frames are shared with up to three helper
+// threads, which touch the destination while the GPU still works; they end with
+// the call. Through the filter, C4F32 at 1080p (16.6 MB out) 1460 -> 980 us, the
+// shipped architecture at 720p (7.4 MB out) 2060 -> 1880 us.
+class ChunkedDownload {
+ public:
+  ChunkedDownload() = default;
+  ChunkedDownload(const ChunkedDownload&) = delete;
+  ChunkedDownload& operator=(const ChunkedDownload&) = delete;
+  ~ChunkedDownload();
+
+  hipError_t Enqueue(int device, hipStream_t s, void* pinned, const void* dev, size_t bytes);
+  // The staged bytes are the planes' rows, plane after plane. Blocks until they
+  // are all copied; on failure the destination's content is unspecified.
+  hipError_t CopyOut(const std::vector<HostRows>& planes);
+
+ private:
+  std::vector<hipEvent_t> events_;
+  int device_ = 0;
+  const uint8_t* pinned_ = nullptr;
+  size_t bytes_ = 0, chunk_ = 0;
+  int n_chunks_ = 0;
+};
+
+}  // namespace arthip

@@ -2497,6 +2497,16 @@ __device__ __forceinline__ float plane_load(const void* p, int64_t i, int kind) 
   }
 }
 
+// Byte copy between device and pinned host memory (small boundary tensors).
+__global__ void __launch_bounds__(256) copy_kernel(uint8_t* dst, const uint8_t* src, int64_t n) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  const int64_t n16 = n / 16;
+  for (int64_t i = t; i < n16; i += step)
+    reinterpret_cast<u4*>(dst)[i] = reinterpret_cast<const u4*>(src)[i];
+  for (int64_t i = 16 * n16 + t; i < n; i += step) dst[i] = src[i];
+}
+
 __global__ void __launch_bounds__(256) plane_convert(PlaneArgs a) {
 #pragma clang fp contract(off)
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n;
@@ -3060,6 +3070,13 @@ hipError_t launch_zero_border(void* buf, int32_t N, int32_t H, int32_t W, int32_
   if (total == 0) return hipSuccess;
   hipLaunchKernelGGL(zero_border, dim3(grid_for(total, 256)), dim3(256), 0, s,
                      static_cast<uint16_t*>(buf), N, H, W, C, (int32_t)Hp, (int32_t)Wp);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy(void* dst, const void* src, size_t n, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(copy_kernel, dim3(grid_for((int64_t)(n + 15) / 16, 256)), dim3(256), 0, s,
+                     static_cast<uint8_t*>(dst), static_cast<const uint8_t*>(src), (int64_t)n);
   return hipGetLastError();
 }
 

@@ -180,7 +180,7 @@ class Model:
         # The output size follows this frame (a variable-size clip has no fixed one).
         ow, oh = src[0].shape[1] * self.scale_w, src[0].shape[0] * self.scale_h
         od = self.format.dtype
-        outs = [np.zeros((oh, ow + out_row_pad), dtype=od)[:, :ow] for _ in range(self.planes_written)]
+        outs = [np.empty((oh, ow + out_row_pad), dtype=od)[:, :ow] for _ in range(self.planes_written)]
         m = len(outs)
         dp = (ctypes.c_void_p * m)(*[o.ctypes.data for o in outs])
         ds = (ctypes.c_ssize_t * m)(*[o.strides[0] for o in outs])
