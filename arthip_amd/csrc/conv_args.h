@@ -185,6 +185,17 @@ struct HeadPairArgs {
   const float* bias1;  // [32] fp32
 };
 
+// A 32 -> 32 conv and the 32 -> 4 tail with DepthToSpace(2) that reads it
+// (conv3x3_tail_pair): r is the first conv's, with r.out the boundary output
+// [N][1][2 H][2 W] in fp16 or fp32.
+struct TailPairArgs {
+  DirectRowArgs r;
+  const uint16_t* w2;  // the tail's row-packed taps (narrow_packed_halfs)
+  const float* bias2;
+  int32_t act2, do_clip;
+  float clip_lo, clip_hi;
+};
+
 // Elementwise / layout kernels for the ops the conv epilogues do not absorb.
 enum UnaryOp : int32_t { kUnarySigmoid = 0, kUnaryRelu = 1, kUnaryClip = 2 };
 enum BinaryOp : int32_t { kBinaryAdd = 0, kBinaryMul = 1 };

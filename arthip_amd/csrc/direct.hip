@@ -261,6 +261,28 @@ __device__ __forceinline__ void rows_fold(const h8 (&wa)[3][L::KR][OB], const ch
     }
 }
 
+// One input row times the taps of the three kernel rows, each onto its own sums
+// (acc[dy]): the row's values are read from LDS once. C = 32's swizzled rows.
+template <class L, int OB>
+__device__ __forceinline__ void rows_fold_once(const h8 (&wa)[3][L::KR][OB], const char* row, const int (&rb)[L::KR],
+                                               f4 (&acc)[3][L::T][OB]) {
+  constexpr int T = L::T, KR = L::KR;
+  static_assert(L::VO == 4, "no masked values");
+#pragma unroll
+  for (int kc = 0; kc < KR; ++kc) {
+    h8 v[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) v[t] = *reinterpret_cast<const h8*>(row + rb[kc] + 16 * L::PXB * t);
+#pragma unroll
+    for (int dy = 2; dy >= 0; --dy)
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int b = 0; b < OB; ++b)
+          acc[dy][t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[dy][kc][b], v[t], acc[dy][t][b], 0, 0, 0);
+  }
+}
+
 // One staged output row leaves linearly: NS whole-kilobyte stores from lin.
 template <int NS, int AUX>
 __device__ __forceinline__ void rows_store(const char* lin, __amdgpu_buffer_rsrc_t ro, int lane) {
@@ -633,6 +655,219 @@ conv3x3_head_pair(HeadPairArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Tail pair: 32 -> 32 conv, then the 32 -> 4 tail conv with DepthToSpace(2)
+// ---------------------------------------------------------------------------
+//
+// conv3x3_rows whose output rows t do not leave: they go into a second LDS ring
+// (fp16, zero outside the image, which is the tail's padding), and the tail conv
+// reads them from there. Each row is read from LDS once and multiplied by the
+// taps of all three kernel rows, onto the sums of three output rows (conv3x3_rows
+// reads it three times, which here bound the kernel by its LDS reads: the frame
+// below took 48.1 and 128 us).
+// Step i takes input row i, which completes t row i - 2, and t row i - 3, which
+// completes output row i - 5. The tail's nine taps are K = 32 products like the
+// conv's, of which only four rows of A hold a channel (0, 1 in rows 0, 1 and 2, 3
+// in rows 4, 5, taken from the packed taps of conv3x3_tail), so lane (q, j),
+// q < 2, ends with the two values of output row 2 y + q at pixel 2 x: one store
+// per tile, bias, activation and Clip in fp32 before it.
+// Every step issues NI copies (LA rows ahead) and NST stores.
+// The LDS reads and writes of a step, and at small sizes the launch and the fill of
+// a run, bound it. The 32-channel model's frame with conv and tail apart and in
+// one launch: 54.3 -> 47.2 us at 540x960, 155.7 -> 121 at 1080p, 300 -> 220 at
+// 2x1080x1920.
+struct TailPairL : RowsL<32, 2, 0> {
+  static constexpr int OPX = IPX - 4;  // output pixels per segment, at most
+  static constexpr int LA = 3;
+  static constexpr int R = LA + 1;     // input ring slots
+  static constexpr int TR = R * SLOT;  // two t slots
+  static constexpr size_t lds_bytes() { return TR + 2 * SLOT + 256; }  // reads run 128 bytes past a slot
+};
+
+// PACK: the output is aligned for two-element stores.
+template <int ACT1, bool F32, bool PACK>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+conv3x3_tail_pair(TailPairArgs a) {
+  using L = TailPairL;
+  constexpr int T = L::T, KR = L::KR, NI = L::NI, LA = L::LA, R = L::R, OB = 2;
+  constexpr int NST = PACK ? T : 2 * T;
+  constexpr int EB = F32 ? 4 : 2;  // bytes per output element
+  static_assert(LA == 3 && R == 4, "the waits of steps 0 .. LA - 1, slots by mask");
+  extern __shared__ __attribute__((aligned(16))) char rlds[];
+  const int lane = threadIdx.x;
+  const int j = lane & 15;
+  const int q = lane >> 4;
+
+  const int G = gridDim.x;
+  const int slot = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+  const int begin = split_begin(a.r.split, slot);
+  const int end = split_begin(a.r.split, slot + 1);
+  if (begin >= end) return;
+
+  h8 wa[3][KR][OB];
+  h8 wt[3][KR][1];  // the tail's taps
+  f4 bias4[OB];
+  float tb[2];
+  {
+    const h8* wp = reinterpret_cast<const h8*>(a.r.w) + lane;
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+      for (int kc = 0; kc < KR; ++kc)
+#pragma unroll
+        for (int b = 0; b < OB; ++b) wa[dy][kc][b] = wp[((dy * KR + kc) * OB + b) * 64];
+#pragma unroll
+    for (int b = 0; b < OB; ++b) bias4[b] = *reinterpret_cast<const f4*>(a.r.bias + q * 4 * OB + 4 * b);
+    // Packed as [dy][lane (q, dx * 4 + n)][8] (conv3x3_tail's B operand).
+    const bool live = (j & 3) < 2 && j < 6;
+    const int ch = 2 * (j >> 2) + (j & 1);
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx) {
+        const h8 v = reinterpret_cast<const h8*>(a.w2)[dy * 64 + 16 * q + dx * 4 + (live ? ch : 0)];
+        wt[dy][dx][0] = live ? v : h8{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    tb[0] = a.bias2[2 * (q & 1)];
+    tb[1] = a.bias2[2 * (q & 1) + 1];
+  }
+  const int H = a.r.H, W = a.r.W;
+  const uint32_t rowb = (uint32_t)a.r.Wp * L::PXB;
+  const uint32_t img = (uint32_t)a.r.Hp * rowb;
+  const uint32_t lds0 = lds_byte_addr(rlds);
+  int rb[KR];
+#pragma unroll
+  for (int kc = 0; kc < KR; ++kc) rb[kc] = (j + kc) * L::PXB + ((q ^ (((j + kc) >> 1) & 2)) << 4);
+  const int tw = j * L::PXB + ((q ^ ((j >> 1) & 2)) << 4);  // t pixel j, octet q
+
+  for (int it = begin; it < end;) {
+    const uint32_t tt = fdiv((uint32_t)it, a.r.fd_H);
+    const int y0 = it - (int)(tt * (uint32_t)H);
+    const uint32_t nn = fdiv(tt, a.r.fd_seg);
+    const int sg = (int)(tt - nn * (uint32_t)a.r.n_seg);
+    const int n = (int)nn;
+    const int len = min(end - it, H - y0);
+    const int x0 = sg * a.r.seg_w;
+    const int valid = min(a.r.seg_w, W - x0);
+    const char* ib = reinterpret_cast<const char*>(a.r.in) + (int64_t)n * img;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)ib, (short)0, (int)img, 0x00020000);
+    char* const ob = reinterpret_cast<char*>(a.r.out) + (int64_t)n * 4 * H * W * EB;
+    const __amdgpu_buffer_rsrc_t ro =
+        __builtin_amdgcn_make_buffer_rsrc((void*)ob, (short)0, (int)((uint32_t)4 * H * W * EB), 0x00020000);
+    // Ring pixel i is padded column x0 - 1 + i, t pixel p image column x0 - 1 + p.
+    uint32_t doff[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int px = (1024 / L::PXB) * i + (lane >> 2);
+      const int col = x0 - 1 + px;
+      const uint32_t src = (uint32_t)(col * L::PXB + (((lane & 3) ^ ((lane >> 3) & 2)) << 4));
+      doff[i] = col >= 0 && col < a.r.Wp && px < valid + 4 ? src : kOob;
+    }
+    uint32_t cmask[T], ooff[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int x = x0 - 1 + 16 * t + j;
+      cmask[t] = x >= 0 && x < W ? ~0u : 0u;
+      const int o = 16 * t + j;
+      ooff[t] = q < 2 && o < valid ? (uint32_t)(q * 2 * W + 2 * (x0 + o)) * EB : kOob;
+    }
+    // Input row i of the run (padded row y0 - 1 + i) into ring slot s.
+    auto issue_row = [&](int i, int s) {
+      const int pr = y0 - 1 + i;
+      const uint32_t rofs = pr >= 0 && pr < a.r.Hp && i <= len + 3 ? (uint32_t)pr * rowb : kOob;  // uniform
+#pragma unroll
+      for (int c = 0; c < NI; ++c)
+        dma16_buf(lds0 + (uint32_t)(s * L::SLOT + 1024 * c), rs, (doff[c] | rofs) >= kOob ? kOob : doff[c] + rofs);
+    };
+#pragma unroll
+    for (int i = 0; i < LA; ++i) issue_row(i, i);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the taps, see conv3x3_rows
+    // Sums of three rows each: A[2] the oldest, completed by this step's row.
+    const f4 z = {0, 0, 0, 0};
+    f4 A[3][T][OB], O[3][T][1];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        A[d][t][0] = A[d][t][1] = z;
+        O[d][t][0] = z;
+      }
+    }
+#pragma unroll 1
+    for (int i = 0; i < len + 5; ++i) {
+      // Input row i has landed.
+      if (i >= LA)
+        wait_vmcnt<(LA - 1) * NI + LA * NST>();
+      else if (i == 0)
+        wait_vmcnt<(LA - 1) * NI>();
+      else if (i == 1)
+        wait_vmcnt<(LA - 1) * NI + NST>();
+      else
+        wait_vmcnt<(LA - 1) * NI + 2 * NST>();
+      issue_row(i + LA, (i + LA) & (R - 1));
+      // Output row i - 5 from t rows up to i - 3, in the slot of the step before.
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        O[2][t][0] = O[1][t][0];
+        O[1][t][0] = O[0][t][0];
+        O[0][t][0] = z;
+      }
+      rows_fold_once<L, 1>(wt, rlds + L::TR + ((i + 1) & 1) * L::SLOT, rb, O);
+      if (i < len + 4) {  // uniform: t row i - 2
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int b = 0; b < OB; ++b) {
+            A[2][t][b] = A[1][t][b];
+            A[1][t][b] = A[0][t][b];
+            A[0][t][b] = bias4[b];
+          }
+        rows_fold_once<L, OB>(wa, rlds + (i & (R - 1)) * L::SLOT, rb, A);
+        const int y = y0 + i - 3;
+        const uint32_t rmask = y >= 0 && y < H ? ~0u : 0u;  // uniform
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          const h4 r0 = strip_act4<ACT1>(A[2][t][0]), r1 = strip_act4<ACT1>(A[2][t][1]);
+          const u4 m = {rmask & cmask[t], rmask & cmask[t], rmask & cmask[t], rmask & cmask[t]};
+          *reinterpret_cast<u4*>(rlds + L::TR + (i & 1) * L::SLOT + tw + 16 * L::PXB * t) =
+              __builtin_bit_cast(u4, __builtin_shufflevector(r0, r1, 0, 1, 2, 3, 4, 5, 6, 7)) & m;
+        }
+      }
+      const uint32_t orow = i >= 5 ? (uint32_t)(y0 + i - 5) * (uint32_t)(4 * W) * EB : kOob;  // uniform
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        float v[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          v[e] = apply_act(O[2][t][0][e] + tb[e], a.act2);
+          if (a.do_clip) v[e] = apply_clip(v[e], a.clip_lo, a.clip_hi);
+        }
+        const uint32_t off = (ooff[t] | orow) >= kOob ? kOob : ooff[t] + orow;
+        if constexpr (F32) {
+          const u2 b = {__builtin_bit_cast(uint32_t, v[0]), __builtin_bit_cast(uint32_t, v[1])};
+          if constexpr (PACK) {
+            __builtin_amdgcn_raw_buffer_store_b64(b, ro, off, 0, 0);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b32(b[0], ro, off, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(b[1], ro, off + 4, 0, 0);
+          }
+        } else {
+          const _Float16 b0 = (_Float16)v[0], b1 = (_Float16)v[1];
+          if constexpr (PACK) {
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, h2{b0, b1}), ro, off, 0, 0);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, b0), ro, off, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, b1), ro, off + 2, 0, 0);
+          }
+        }
+      }
+    }
+    it += len;
+  }
+  wait_vmcnt<0>();  // no copy into LDS outlives the workgroup
+}
+
+// ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
 
@@ -833,6 +1068,45 @@ hipError_t launch_head_pair(const DirectArgs& head, const WinoArgs& conv, hipStr
   const hipError_t e = rows_grid(fn, a.r, 64, HeadPairL::lds_bytes(), 8, 2, &blocks);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(blocks), dim3(64), HeadPairL::lds_bytes(), s, a);
+  return hipGetLastError();
+}
+
+// The conv alone would run conv3x3_rows and the tail conv3x3_tail.
+bool tail_pair_eligible(int64_t N, int64_t H, int64_t W, bool fp32) {
+  const int64_t out = 4 * H * W * (fp32 ? 4 : 2);
+  return !tiny32(N, H, W) && fits32(N, H, W, 32, TailPairL::OPX) && out < (int64_t)1 << 31;
+}
+
+hipError_t launch_tail_pair(const WinoArgs& conv, const WinoArgs& tail, hipStream_t s) {
+  const bool f32 = tail.epi.out_kind == kOutNchwF32;
+  if (!tail_pair_eligible(conv.N, conv.H, conv.W, f32) || conv.C != 32 || conv.M != 32 || tail.C != 32 ||
+      tail.M != 4 || tail.epi.dts_b != 2 || (!f32 && tail.epi.out_kind != kOutNchwF16) ||
+      conv.epi.skip0 != nullptr || conv.epi.skip1 != nullptr || tail.epi.skip0 != nullptr ||
+      tail.epi.skip1 != nullptr || conv.epi.do_clip || !aligned16(conv.in))
+    return hipErrorInvalidValue;
+  TailPairArgs a{};
+  a.r = row_args(conv, TailPairL::OPX);
+  a.r.out = static_cast<uint16_t*>(tail.epi.out);
+  a.w2 = tail.u + winograd_u_halfs(32, 4);
+  a.bias2 = tail.epi.bias;
+  a.act2 = tail.epi.act;
+  a.do_clip = tail.epi.do_clip;
+  a.clip_lo = tail.epi.clip_lo;
+  a.clip_hi = tail.epi.clip_hi;
+  using Fn = void (*)(TailPairArgs);
+  auto pick = [&](auto f32_tag, auto pack_tag) -> Fn {
+    constexpr bool F = decltype(f32_tag)::value != 0, P = decltype(pack_tag)::value != 0;
+    return conv.epi.act == kActRelu   ? conv3x3_tail_pair<kActRelu, F, P>
+           : conv.epi.act == kActSilu ? conv3x3_tail_pair<kActSilu, F, P>
+                                      : conv3x3_tail_pair<kActNone, F, P>;
+  };
+  const bool pack = reinterpret_cast<uintptr_t>(tail.epi.out) % (f32 ? 8 : 4) == 0;
+  const Fn fn = f32 ? (pack ? pick(IntC<1>{}, IntC<1>{}) : pick(IntC<1>{}, IntC<0>{}))
+                    : (pack ? pick(IntC<0>{}, IntC<1>{}) : pick(IntC<0>{}, IntC<0>{}));
+  unsigned blocks = 0;
+  const hipError_t e = rows_grid(fn, a.r, 64, TailPairL::lds_bytes(), 8, 4, &blocks);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(blocks), dim3(64), TailPairL::lds_bytes(), s, a);
   return hipGetLastError();
 }
 

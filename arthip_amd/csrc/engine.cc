@@ -654,8 +654,53 @@ bool Engine::EnsurePlan(Plan& p, const int64_t in[4], std::string& error, void* 
     return c1 == 1 && m1 == 32 && c2 == 32 && m2 == 32 &&
            head_pair_eligible(sin.n, sin.h, sin.w, graph_.input_fp32);
   };
+  // A 32 -> 32 conv and the final 32 -> 4 conv with DepthToSpace(2), when that is
+  // its only reader (conv3x3_tail_pair).
+  auto tail_at = [&](int i) -> bool {
+    if ((debug_ & kDebugUnfused) || i + 1 >= nops || i == fused_in_op) return false;
+    if (!direct_out || i + 1 != final_op) return false;
+    const Op& a = ops[i];
+    const Op& b = ops[i + 1];
+    if (a.kind != OpKind::Conv || b.kind != OpKind::Conv || b.in0 != a.out) return false;
+    if (!a.skips.empty() || a.clip || a.dts_b >= 1 || !b.skips.empty() || b.dts_b != 2) return false;
+    if (readers(a.out) != 1) return false;
+    int64_t c1, m1, c2, m2;
+    conv_cm(a, c1, m1);
+    conv_cm(b, c2, m2);
+    const Shape si = shapes.at(a.in0);
+    return c1 == 32 && m1 == 32 && c2 == 32 && m2 == 4 &&
+           tail_pair_eligible(si.n, si.h, si.w, graph_.output_fp32);
+  };
   for (int i = 0; i < nops; ++i) {
     const Op& op = ops[i];
+    if (tail_at(i)) {
+      const Op& op2 = ops[i + 1];
+      const Shape si = shapes.at(op.in0);
+      // The conv's output is never written; its place in the plan stays, and
+      // with it the input sizes that a scratch plan takes.
+      if (!alloc(op.out, shapes.at(op.out), i)) return fail();
+      Step st;
+      st.kind = StepKind::TailPair;
+      st.op = i;
+      st.op2 = i + 1;
+      st.in = tbuf.at(op.in0);
+      st.out = kBoundaryOut;
+      st.N = (int32_t)si.n; st.H = (int32_t)si.h; st.W = (int32_t)si.w; st.C = 32; st.M = 4;
+      st.wbuf = op_wbuf_.at(i);
+      st.bbuf = op_bbuf_.at(i);
+      st.wbuf2 = op_wbuf_.at(i + 1);
+      st.bbuf2 = op_bbuf_.at(i + 1);
+      st.epi.act = op.act;
+      st.act2 = op2.act;
+      st.epi.out_kind = out_kind_boundary;
+      st.epi.dts_b = 2;
+      st.epi.do_clip = op2.clip ? 1 : 0;
+      st.epi.clip_lo = op2.clip_lo;
+      st.epi.clip_hi = op2.clip_hi;
+      p.steps.push_back(st);
+      ++i;
+      continue;
+    }
     if (pair_at(i)) {
       const Op& op2 = ops[i + 1];
       if (!alloc(op2.out, shapes.at(op2.out), i)) return fail();
@@ -1008,6 +1053,23 @@ bool Engine::Enqueue(const Plan& p, const void* in_dev, void* out_dev, hipStream
         e = launch_head_pair(h, c, s);
         break;
       }
+      case StepKind::TailPair: {
+        WinoArgs c{};
+        c.in = static_cast<const uint16_t*>(ptr(st.in));
+        c.u = static_cast<const uint16_t*>(wbufs_[st.wbuf].ptr);
+        c.epi.bias = static_cast<const float*>(wbufs_[st.bbuf].ptr);
+        c.epi.act = st.epi.act;
+        c.N = st.N; c.H = st.H; c.W = st.W; c.C = 32; c.M = 32;
+        WinoArgs t{};
+        t.u = static_cast<const uint16_t*>(wbufs_[st.wbuf2].ptr);
+        t.epi = st.epi;
+        t.epi.act = st.act2;
+        t.epi.bias = static_cast<const float*>(wbufs_[st.bbuf2].ptr);
+        t.epi.out = ptr(st.out);
+        t.N = st.N; t.H = st.H; t.W = st.W; t.C = 32; t.M = 4;
+        e = launch_tail_pair(c, t, s);
+        break;
+      }
       case StepKind::Eltwise: {
         EltArgs a{};
         a.a = static_cast<const uint16_t*>(ptr(st.in));
@@ -1135,6 +1197,10 @@ std::string Engine::StepName(const Step& st) const {
       break;
     case StepKind::HeadPair:
       os << "head_pair C1 M32" << acts[st.epi.act] << ", C32 M32" << acts[st.act2];
+      break;
+    case StepKind::TailPair:
+      os << "tail_pair C32 M32" << acts[st.epi.act] << ", C32 M4" << acts[st.act2] << " +dts2";
+      if (st.epi.do_clip) os << " +clip";
       break;
     case StepKind::Eltwise: os << "eltwise op" << st.elt_op << (st.binary ? " binary" : ""); break;
     case StepKind::DepthToSpace: os << "depth_to_space b" << st.dts_b; break;

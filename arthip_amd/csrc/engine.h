@@ -40,7 +40,7 @@ enum DebugFlag : int {
   kDebugPoison = 1,       // before each run, fill every activation interior with fp16 NaN
   kDebugSyncEach = 2,     // synchronize the launch stream after every launch
   kDebugDump = 4,         // write each launch's inputs and output (first two runs)
-  kDebugUnfused = 8,      // run every conv as its own launch (no residual-block fusion)
+  kDebugUnfused = 8,      // run every conv as its own launch (no fused blocks or pairs)
   kDebugTrace = 16,       // "[run]" lines: enter, plan ready, each launch, done / fail
   kDebugHostProfile = 32, // "[hipprof]" host time spans of each run
   kDebugDumpOps = 64,     // "[dump]" line per launch: its buffers, addresses and sizes
@@ -55,6 +55,7 @@ enum class StepKind {
   ConvDirect,
   ConvBlock,  // two 64 -> 64 convs fused (winograd_block): op, op2
   HeadPair,   // a 1 -> 32 head conv and the 32 -> 32 conv after it: op, op2
+  TailPair,   // a 32 -> 32 conv and the 32 -> 4 tail after it: op, op2
   Eltwise,
   DepthToSpace,
   OutputConvert
@@ -69,12 +70,12 @@ constexpr int kNoBuffer = -1;
 struct Step {
   StepKind kind = StepKind::ConvWinograd;
   int op = -1;   // index into Graph::ops (-1 for IO steps)
-  int op2 = -1;  // ConvBlock, HeadPair: the second conv
+  int op2 = -1;  // ConvBlock, HeadPair, TailPair: the second conv
   int in = kNoBuffer, in2 = kNoBuffer, out = kNoBuffer;
   int skip[2] = {kNoBuffer, kNoBuffer};
   int wbuf = kNoBuffer, bbuf = kNoBuffer;  // packed weights / padded bias (weight cache)
   int wbuf2 = kNoBuffer, bbuf2 = kNoBuffer;  // the second conv's
-  int32_t act2 = kActNone;  // HeadPair: the second conv's activation
+  int32_t act2 = kActNone;  // HeadPair, TailPair: the second conv's activation
   // Geometry of the step's input (NHWC) and channel counts.
   int32_t N = 0, H = 0, W = 0, C = 0, M = 0;
   Epilogue epi{};  // conv epilogue (pointers resolved per run)

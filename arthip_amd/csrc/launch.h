@@ -78,6 +78,11 @@ hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s);
 // 32 -> 32 conv (no residual input) that alone reads it, in one launch.
 bool head_pair_eligible(int64_t N, int64_t H, int64_t W, bool fp32);
 hipError_t launch_head_pair(const DirectArgs& head, const WinoArgs& conv, hipStream_t s);
+// A 32 -> 32 conv (no residual input) and the 32 -> 4 tail conv with
+// DepthToSpace(2) that alone reads it, writing the NCHW boundary output (fp32:
+// its type), in one launch.
+bool tail_pair_eligible(int64_t N, int64_t H, int64_t W, bool fp32);
+hipError_t launch_tail_pair(const WinoArgs& conv, const WinoArgs& tail, hipStream_t s);
 hipError_t launch_eltwise(EltArgs a, bool binary, hipStream_t s);
 hipError_t launch_dts(DtsArgs a, hipStream_t s);
 hipError_t launch_input_convert(IoArgs a, hipStream_t s);

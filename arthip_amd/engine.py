@@ -228,7 +228,7 @@ class Engine:
         (hip_engine.cc:1310-1349): POISON fills every activation interior with
         fp16 NaN before each run, SYNC_EACH synchronizes after every launch, DUMP
         writes each launch's inputs and output under dump_dir (first two runs),
-        UNFUSED runs every conv as its own launch (no residual-block fusion).
+        UNFUSED runs every conv as its own launch (no fused blocks or pairs).
         Host-side lines to the engine's log (set_log): TRACE (VSHIP_TRACE),
         HOST_PROFILE (HIP_PROFILE), DUMPOPS (HIP_DUMPOPS), PLAN (VSHIP_DEBUG)."""
         d = str(dump_dir).encode() if dump_dir is not None else None

@@ -406,8 +406,8 @@ def launch_work(spec, steps, px: int):
             # The fused block runs F(2,3) along x, the kernel rows direct: 6 of
             # the 9 products per output and channel pair.
             out.append({"bytes": b, "flops_direct": fd, "flops_wino": fd * 6 / 9, "convs": 2})
-        elif name.startswith("head_pair"):
-            # A head conv and the conv after it, the tensor between them on chip.
+        elif name.startswith(("head_pair", "tail_pair")):
+            # Two convs, the tensor between them on chip.
             (c1, m1), _ = convs[ci]
             (c2, m2), _ = convs[ci + 1]
             ci += 2

@@ -145,8 +145,10 @@ int arthip_engine_profile_read(arthip_engine* eng, int max_steps, double* total_
  *   fp16 layout of arthip_padded_dims, boundary tensors as given).
  * - UNFUSED (no environment switch): every conv runs as its own launch; by
  *   default a 64 -> 64 conv whose output only the next 64 -> 64 conv reads
- *   runs fused with it (arthip_conv3x3_block_f16_nhwc), which agrees with
- *   separate launches to fp16 rounding. Changing it drops the cached plans.
+ *   runs fused with it (arthip_conv3x3_block_f16_nhwc), and a 32-channel
+ *   model's head with the conv after it and its last conv with the tail;
+ *   they agree with separate launches to fp16 rounding. Changing it drops the
+ *   cached plans.
  * Host-side lines, written to the engine's log (stderr, or the file given to
  * arthip_engine_set_log):
  * - TRACE (VSHIP_TRACE=1; hip_engine.cc:1280-1298,1421-1425,1619): per run
