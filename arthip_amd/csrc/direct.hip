@@ -466,7 +466,7 @@ conv3x3_rows(DirectRowArgs a) {
 // k .. k + 2; the input of the row after that is requested a step ahead. Head
 // pixels outside the image are zero: the second conv's padding.
 // The output's write stream and the launch bound it. At 540x960: 11 us for the
-// head and 17 for the conv apart, 18 here; the 32-channel model's frame 62.7 -> 54.7
+// head and 17 for the conv apart, 20 here; the 32-channel model's frame 62.7 -> 54.7
 // us, at 2x1080x1920 390 -> 301.
 struct HeadPairL : RowsL<32, 2, 0> {
   static constexpr int R = 4;
