@@ -1282,6 +1282,8 @@ bool Engine::Run(const void* in_host, const int64_t in[4], void* out_host, size_
   if (!Enqueue(plan_, in_stage_dev_, out_stage_dev_, stream_, error)) return false;
   rl.Launched();
   const bool small = out_bytes <= kKernelCopyBytes;
+  const std::vector<HostRows> rows{
+      HostRows{static_cast<uint8_t*>(out_host), static_cast<ptrdiff_t>(out_bytes), out_bytes, 1}};
   e = small ? launch_copy(out_pinned_, out_stage_dev_, out_bytes, stream_)
             : download_.Enqueue(device_, stream_, out_pinned_, out_stage_dev_, out_bytes);
   if (e != hipSuccess) {
@@ -1290,7 +1292,7 @@ bool Engine::Run(const void* in_host, const int64_t in[4], void* out_host, size_
   }
   if (!small) {
     // Copied out as it arrives; the synchronize below then only reports errors.
-    e = download_.CopyOut({HostRows{static_cast<uint8_t*>(out_host), static_cast<ptrdiff_t>(out_bytes), out_bytes, 1}});
+    e = download_.CopyOut(rows);
     if (e != hipSuccess) {
       error = HipErr("HIP output download", e);
       return false;

@@ -3,7 +3,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
 #include <thread>
 
 namespace arthip {
@@ -109,8 +108,8 @@ hipError_t ChunkedDownload::CopyOut(const std::vector<HostRows>& planes) {
         else
           work(started);
       });
-    } catch (const std::system_error&) {
-      break;  // no thread to be had: the caller copies that part too
+    } catch (...) {
+      break;  // no thread or no memory for one: the caller copies that part too
     }
   }
   work(0);

@@ -54,14 +54,19 @@ static void direct_rows_pack(const float* w, int M, int C, uint16_t* out) {
   const bool head = direct_head_shape(C, M);
   for (int m = 0; m < M; ++m) {
     const int b = m % (4 * n_ob) / 4, i = m / (4 * n_ob) * 4 + m % 4;  // A row i of block b
-    for (int dy = 0; dy < 3; ++dy)
-      for (int k = 0; k < 3 * C; ++k) {
-        const float v = w[(static_cast<size_t>(m) * C + k % C) * 9 + dy * 3 + k / C];
-        const size_t idx =
-            head ? (static_cast<size_t>(b) * 64 + dy * 16 + i) * 16 + k
-                 : (((static_cast<size_t>(dy) * kr + k / 32) * n_ob + b) * 64 + k % 32 / 8 * 16 + i) * 8 + k % 8;
-        out[idx] = f32_to_f16(v);
-      }
+    const float* wm = w + static_cast<size_t>(m) * C * 9;
+    for (int dy = 0; dy < 3; ++dy) {
+      // Value k = dx * C + c of the row at slot q = k / 8 (of four per product), k % 8.
+      uint16_t* const row = head ? out + (static_cast<size_t>(b) * 64 + dy * 16 + i) * 16
+                                 : out + ((static_cast<size_t>(dy) * kr * n_ob + b) * 64 + i) * 8;
+      int k = 0;
+      for (int dx = 0; dx < 3; ++dx)
+        for (int c = 0; c < C; ++c, ++k) {
+          const size_t at = head ? static_cast<size_t>(k)
+                                 : static_cast<size_t>(k >> 5) * n_ob * 512 + ((k >> 3) & 3) * 128 + (k & 7);
+          row[at] = f32_to_f16(wm[c * 9 + dy * 3 + dx]);
+        }
+    }
   }
 }
 

@@ -363,7 +363,9 @@ size_t arthip_conv3x3_bias_len(int M);
 /* Host-side filter transform, done once per layer: the Winograd
  * U = G g G^T for C > 1 (hip_engine.cc:972-1018), a tap relayout for C == 1
  * (hip_engine.cc:925-971). w_oihw holds fp16 bits [M][C][3][3]; bias holds M
- * fp16 values or is NULL. Outputs go to host buffers of the sizes above. */
+ * fp16 values or is NULL. Outputs go to host buffers of the sizes above. Their
+ * layout and size belong to this version of the library: pack with the library
+ * that runs the conv rather than keeping packed buffers across versions. */
 int arthip_conv3x3_pack(const uint16_t* w_oihw, const uint16_t* bias, int M, int C,
                         uint16_t* packed, size_t packed_cap, float* bias_out, size_t bias_cap);
 
