@@ -1270,6 +1270,16 @@ bool Engine::Run(const void* in_host, const int64_t in[4], void* out_host, size_
       return false;
     }
   }
+  const std::vector<HostRows> rows{
+      HostRows{static_cast<uint8_t*>(out_host), static_cast<ptrdiff_t>(out_bytes), out_bytes, 1}};
+  // Left by a failure, whatever is already queued ends first: the next run
+  // writes the staging, and another shape frees it.
+  struct Drain {
+    hipStream_t s;
+    ~Drain() {
+      if (s) (void)hipStreamSynchronize(s);
+    }
+  } drain{stream_};
   std::memcpy(in_pinned_, in_host, in_bytes);
   e = in_bytes <= kKernelCopyBytes
           ? launch_copy(in_stage_dev_, in_pinned_, in_bytes, stream_)
@@ -1282,8 +1292,6 @@ bool Engine::Run(const void* in_host, const int64_t in[4], void* out_host, size_
   if (!Enqueue(plan_, in_stage_dev_, out_stage_dev_, stream_, error)) return false;
   rl.Launched();
   const bool small = out_bytes <= kKernelCopyBytes;
-  const std::vector<HostRows> rows{
-      HostRows{static_cast<uint8_t*>(out_host), static_cast<ptrdiff_t>(out_bytes), out_bytes, 1}};
   e = small ? launch_copy(out_pinned_, out_stage_dev_, out_bytes, stream_)
             : download_.Enqueue(device_, stream_, out_pinned_, out_stage_dev_, out_bytes);
   if (e != hipSuccess) {
@@ -1302,6 +1310,7 @@ bool Engine::Run(const void* in_host, const int64_t in[4], void* out_host, size_
     error = HipErr("HIP stream synchronize", e);
     return false;
   }
+  drain.s = nullptr;
   rl.Back();
   if (small) std::memcpy(out_host, out_pinned_, out_bytes);
   return rl.Done(out_host);

@@ -53,6 +53,12 @@ ChunkedDownload::~ChunkedDownload() {
 }
 
 hipError_t ChunkedDownload::Enqueue(int device, hipStream_t s, void* pinned, const void* dev, size_t bytes) {
+  const hipError_t r = Send(device, s, pinned, dev, bytes);
+  if (r != hipSuccess) (void)hipStreamSynchronize(s);
+  return r;
+}
+
+hipError_t ChunkedDownload::Send(int device, hipStream_t s, void* pinned, const void* dev, size_t bytes) {
   const size_t want = std::min(kMaxChunks, std::max<size_t>(1, bytes / kMinChunk));
   const size_t chunk = ((bytes + want - 1) / want + kPage - 1) / kPage * kPage;
   events_.reserve(kMaxChunks);
@@ -63,6 +69,7 @@ hipError_t ChunkedDownload::Enqueue(int device, hipStream_t s, void* pinned, con
     events_.push_back(e);
   }
   device_ = device;
+  stream_ = s;
   pinned_ = static_cast<const uint8_t*>(pinned);
   bytes_ = bytes;
   chunk_ = chunk;
@@ -116,7 +123,10 @@ hipError_t ChunkedDownload::CopyOut(const std::vector<HostRows>& planes) {
   for (size_t w = started; w < parts; ++w) work(w);
   for (std::thread& t : helpers)
     if (t.joinable()) t.join();
-  return static_cast<hipError_t>(failed.load());
+  const hipError_t r = static_cast<hipError_t>(failed.load());
+  // Chunks that nobody waited for may still be on their way into the staging.
+  if (r != hipSuccess) (void)hipStreamSynchronize(stream_);
+  return r;
 }
 
 }  // namespace arthip

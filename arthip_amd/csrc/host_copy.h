@@ -39,14 +39,19 @@ class ChunkedDownload {
   ChunkedDownload& operator=(const ChunkedDownload&) = delete;
   ~ChunkedDownload();
 
+  // Both wait for the stream before they report a failure, so that no chunk
+  // still writes the staging, which the caller may then reuse or free.
   hipError_t Enqueue(int device, hipStream_t s, void* pinned, const void* dev, size_t bytes);
   // The staged bytes are the planes' rows, plane after plane. Blocks until they
   // are all copied; on failure the destination's content is unspecified.
   hipError_t CopyOut(const std::vector<HostRows>& planes);
 
  private:
+  hipError_t Send(int device, hipStream_t s, void* pinned, const void* dev, size_t bytes);
+
   std::vector<hipEvent_t> events_;
   int device_ = 0;
+  hipStream_t stream_ = nullptr;
   const uint8_t* pinned_ = nullptr;
   size_t bytes_ = 0, chunk_ = 0;
   int n_chunks_ = 0;
