@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <numeric>
 #include <string>
 
 #include "conv_args.h"
@@ -20,18 +21,20 @@ FastDiv make_fastdiv(uint32_t d);
 
 // Ranges of n_items work items (strips of strip_len items) over `slots`
 // workgroups (below 2^15). `fill` is what entering another strip costs a
-// workgroup, in items; strips are padded by it unless the longest unpadded range
-// with the strips that it enters is no longer than the longest padded one: where
-// the slots are a multiple of the strips (1080p: 256 and 64) no range enters any.
+// workgroup, in items. With strips padded by it no range costs more than the
+// padded total over the slots, rounded up. Without, slot s starts
+// strip_len t / slots items into a strip, t = s strips mod slots, a multiple of
+// gcd(strips, slots): the range with the largest t enters the most strips. The
+// strips are padded where their bound is no higher than that range's cost, so
+// never to a longer longest range (1080p on 64 strips and 256 slots: no range
+// enters any, unpadded).
 inline ItemSplit make_split(int32_t n_items, int32_t slots, int32_t strip_len, int32_t fill) {
   const int64_t strips = n_items / strip_len;
   const int64_t padded = n_items + strips * fill;
-  const int64_t longest = (static_cast<int64_t>(n_items) + slots - 1) / slots;
-  const int64_t enters = slots % strips == 0   ? 0
-                         : strips % slots == 0 ? strips / slots - 1
-                                               : (longest + strip_len - 2) / strip_len;
+  const int64_t last_t = slots - std::gcd(strips, static_cast<int64_t>(slots));
+  const int64_t enters = ((strip_len * last_t + n_items) / slots - 1) / strip_len;
   const bool pad = padded < static_cast<int64_t>(1) << 31 &&
-                   (padded + slots - 1) / slots < longest + enters * fill;
+                   (padded + slots - 1) / slots <= n_items / slots + enters * fill;
   const int32_t total = pad ? static_cast<int32_t>(padded) : n_items;
   ItemSplit s{};
   s.pad = pad ? fill : 0;
