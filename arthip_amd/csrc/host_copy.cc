@@ -2,7 +2,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <mutex>
 #include <thread>
 
 namespace arthip {
@@ -88,14 +90,31 @@ hipError_t ChunkedDownload::Send(int device, hipStream_t s, void* pinned, const 
 hipError_t ChunkedDownload::CopyOut(const std::vector<HostRows>& planes) {
   const size_t parts = std::min(kMaxThreads, static_cast<size_t>(std::max(n_chunks_, 1)));
   std::atomic<int> failed{hipSuccess};
+  // Waiting for an event keeps a core busy, so until the first chunk is there,
+  // which is most of a frame's GPU time, only the caller does; the helpers sleep.
+  std::mutex mu;
+  std::condition_variable cv;
+  bool first_seen = false;
+  auto first_done = [&] {
+    {
+      std::lock_guard<std::mutex> g(mu);
+      first_seen = true;
+    }
+    cv.notify_all();
+  };
   // Chunks w, w + parts, ...: whole chunks, so that no two threads fault the
   // same (huge) page of the destination at once, and nobody touches bytes that
   // another thread copies.
   auto work = [&](size_t w) {
     for (size_t k = w; k < static_cast<size_t>(n_chunks_); k += parts)
       for_rows(planes, k * chunk_, std::min((k + 1) * chunk_, bytes_), [](uint8_t* d, size_t, size_t n) { touch(d, n); });
+    if (w != 0) {
+      std::unique_lock<std::mutex> g(mu);
+      cv.wait(g, [&] { return first_seen; });
+    }
     for (size_t k = w; k < static_cast<size_t>(n_chunks_); k += parts) {
       const hipError_t r = hipEventSynchronize(events_[k]);
+      if (k == 0) first_done();
       if (r != hipSuccess) {
         failed.store(r);
         return;

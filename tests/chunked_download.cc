@@ -2,10 +2,12 @@
 // stream land only when something waits for them. Each scenario makes one call
 // fail; the download must not report the failure while a chunk that was sent
 // could still write the staging buffer. argv[1]: scenario.
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "host_copy.h"
@@ -26,6 +28,8 @@ int copies_sent = 0;
 int fail_copy = -1;
 size_t fail_event = 0;  // 1-based, as handed out
 bool fail_device = false;
+bool slow_frame = false;  // the frame takes a while until its first chunk is there
+int early_waits = 0;      // waits for later chunks begun before that
 
 void land(size_t upto) {
   for (; landed < upto; ++landed) std::memcpy(queued[landed].dst, queued[landed].src, queued[landed].n);
@@ -54,7 +58,9 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
   return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
+  if (slow_frame && reinterpret_cast<size_t>(e) == 1) std::this_thread::sleep_for(std::chrono::milliseconds(300));
   std::lock_guard<std::mutex> g(mu);
+  if (reinterpret_cast<size_t>(e) != 1 && !landed) ++early_waits;
   if (reinterpret_cast<size_t>(e) == fail_event) return hipErrorUnknown;
   land(recorded[reinterpret_cast<size_t>(e) - 1]);
   return hipSuccess;
@@ -76,6 +82,7 @@ int main(int argc, char** argv) {
   if (what == "copy") fail_copy = 2;
   if (what == "first_wait") fail_event = 1;
   if (what == "last_wait") fail_event = 4;
+  slow_frame = what == "slow";
   fail_device = what == "device";  // in the helper threads
 
   arthip::ChunkedDownload d;
@@ -91,6 +98,7 @@ int main(int argc, char** argv) {
                    arthip::HostRows{out.data(), static_cast<ptrdiff_t>(rest), rest, 1}});
   std::printf("status %d queued %zu landed %zu\n", static_cast<int>(e), queued.size(), landed);
   if (e != hipSuccess) return landed == queued.size() ? 2 : 1;
+  if (slow_frame && early_waits != 0) return 1;
   for (int y = 0; y < rows; ++y)
     if (std::memcmp(&strided[static_cast<size_t>(y) * 1100], &dev[y * row], row) != 0) return 1;
   return std::memcmp(out.data(), &dev[rows * row], rest) == 0 ? 0 : 1;
