@@ -998,14 +998,7 @@ hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s) {
 // Output pixels of a conv3x3_rows segment.
 static int rows_segment(int C) { return C % 16 == 0 ? RowsL<16, 1, 0>::OPX : RowsL<24, 1, 0>::OPX; }
 
-// 32 -> 32 convs of up to 4096 pixels stay on winograd_strip. Both kernels take
-// about a launch's latency there (36x52: 3.4 us here, 3.8 there), and the
-// models' tests compare such a frame's fp32 and fp16 outputs by errors that
-// they expect to lie above the output's own rounding, as Winograd's do.
-static bool tiny32(int64_t N, int64_t H, int64_t W) { return N * H * W <= 4096; }
-
 bool conv_rows_eligible(const WinoArgs& w) {
-  if (w.C == 32 && w.M == 32 && tiny32(w.N, w.H, w.W)) return false;
   const int64_t cm = w.C > w.M ? w.C : w.M;
   return inner_epilogue(w) && direct_rows_shape(w.C, w.M) && aligned16(w.in) &&
          aligned16(w.epi.out) && aligned16(w.epi.skip0) && aligned16(w.epi.skip1) &&
@@ -1040,7 +1033,7 @@ hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s) {
 // The conv alone would run conv3x3_rows, and the head direct_conv_c1_mfma on the
 // boundary input: the pair gives the same bits as the two.
 bool head_pair_eligible(int64_t N, int64_t H, int64_t W, bool fp32) {
-  return !tiny32(N, H, W) && fits32(N, H, W, 32, HeadPairL::OPX) && head_reads_boundary_input(N, H, W, 32, fp32);
+  return fits32(N, H, W, 32, HeadPairL::OPX) && head_reads_boundary_input(N, H, W, 32, fp32);
 }
 
 hipError_t launch_head_pair(const DirectArgs& head, const WinoArgs& conv, hipStream_t s) {
@@ -1074,7 +1067,7 @@ hipError_t launch_head_pair(const DirectArgs& head, const WinoArgs& conv, hipStr
 // The conv alone would run conv3x3_rows and the tail conv3x3_tail.
 bool tail_pair_eligible(int64_t N, int64_t H, int64_t W, bool fp32) {
   const int64_t out = 4 * H * W * (fp32 ? 4 : 2);
-  return !tiny32(N, H, W) && fits32(N, H, W, 32, TailPairL::OPX) && out < (int64_t)1 << 31;
+  return fits32(N, H, W, 32, TailPairL::OPX) && out < (int64_t)1 << 31;
 }
 
 hipError_t launch_tail_pair(const WinoArgs& conv, const WinoArgs& tail, hipStream_t s) {

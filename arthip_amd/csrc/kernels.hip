@@ -2627,7 +2627,8 @@ StripKernel strip_kernel_act(int act, int nskip) {
 
 // C == M in {32, 64, 96} with the fast epilogue: winograd_strip covers 64
 // channels with residual inputs and the 32-channel convs that conv3x3_rows
-// leaves, the row pipes and winograd_pipe the rest.
+// does not take (buffers off 16 bytes, images of 2 GiB and more), the row pipes
+// and winograd_pipe the rest.
 bool strip_eligible(const WinoArgs& a) {
   const bool fast_epi = a.epi.out_kind == kOutPadded && a.epi.dts_b < 2 && !a.epi.do_clip &&
                         (a.epi.act == kActNone || a.epi.act == kActRelu ||

@@ -397,7 +397,11 @@ def test_fp32_model_runs_the_fp16_network(builder, hw):
     fp16 network: against the fp16 model on the same (fp16-representable)
     input, the fp32 output is the fp16 output before its final rounding, so the
     two differ by at most half an fp16 ulp; and it is within the same bound of
-    the oracle on the fp16 model as the fp16 engine output is."""
+    the oracle on the fp16 model as the fp16 engine output is, up to that
+    rounding. Where the engine meets the oracle's fp16 output almost exactly
+    (c4f32), s16 is below the rounding that the fp32 output does not have:
+    rms(y32 - want) <= rms(y16 - want) + rms(y32 - y16), and the last term is
+    at most the rms of a uniform error of half an ulp, half_ulp / sqrt(3)."""
     spec = builder(seed=0)
     wide = models.widen_to_fp32(spec)
     h, w = hw
@@ -414,7 +418,8 @@ def test_fp32_model_runs_the_fp16_network(builder, hw):
     want = run_model(spec.model, x16)
     s16, s32 = _compare(y16, want), _compare(y32, want)
     print(spec.name, "fp16 model", s16, "fp32 model", s32)
-    assert s32["rel_rms"] <= s16["rel_rms"] * 1.05 + 1e-6
+    rounding = np.sqrt(np.mean(half_ulp ** 2) / 3 / np.mean(np.asarray(want, np.float64) ** 2))
+    assert s32["rel_rms"] <= (s16["rel_rms"] + rounding) * 1.05 + 1e-6
 
 
 @pytest.mark.parametrize("builder,hw", [(models.r8f64, (1, 1)), (models.r8f64, (3, 5)),
