@@ -676,9 +676,6 @@ bool Engine::EnsurePlan(Plan& p, const int64_t in[4], std::string& error, void* 
     if (tail_at(i)) {
       const Op& op2 = ops[i + 1];
       const Shape si = shapes.at(op.in0);
-      // The conv's output is never written; its place in the plan stays, and
-      // with it the input sizes that a scratch plan takes.
-      if (!alloc(op.out, shapes.at(op.out), i)) return fail();
       Step st;
       st.kind = StepKind::TailPair;
       st.op = i;

@@ -138,7 +138,7 @@ def _pair_engines(spec, fp32, x, debug=0):
             e.set_debug(debug)
         alone.set_debug(Engine.DEBUG_UNFUSED)
         got, want = e.build(model).run(x), alone.build(model).run(x)
-        assert "2 launches" in e.describe() and "4 launches" in alone.describe()
+        assert "2 launches, 1 activation buffers" in e.describe() and "4 launches" in alone.describe()
     return got.astype(np.float64), want.astype(np.float64)
 
 
