@@ -15,29 +15,24 @@ inline uint16_t f32_to_f16(float f) {
   std::memcpy(&x, &f, 4);
   const uint32_t sign = (x >> 16) & 0x8000u;
   const uint32_t a = x & 0x7fffffffu;
+  // 2^-14 <= |f| < 2^16, almost every value that is packed: rebias the exponent
+  // and round in the 13 bits that go, a carry into the exponent (at the top: to
+  // inf) being the correct rounding.
+  if (a >= 0x38800000u && a < 0x47800000u)
+    return static_cast<uint16_t>(sign | ((a - 0x38000000u + 0xfffu + ((a >> 13) & 1u)) >> 13));
   if (a >= 0x7f800000u) return static_cast<uint16_t>(sign | 0x7c00u | (a > 0x7f800000u ? 0x200u : 0u));
+  if (a >= 0x47800000u) return static_cast<uint16_t>(sign | 0x7c00u);  // overflow to inf
   // Below half of the smallest subnormal (2^-25): signed zero.
   if (a <= 0x33000000u) return static_cast<uint16_t>(sign);
   const int e = static_cast<int>(a >> 23) - 127;  // unbiased exponent
   uint32_t mant = (a & 0x7fffffu) | 0x800000u;     // 24-bit significand
-  uint32_t bits;
-  if (e < -14) {
-    // Subnormal half: value = mant * 2^(e-23); half ulp is 2^-24.
-    const int shift = -e - 14 + 13;  // 14..24
-    uint32_t q = mant >> shift;
-    const uint32_t rem = mant & ((1u << shift) - 1u);
-    const uint32_t halfway = 1u << (shift - 1);
-    if (rem > halfway || (rem == halfway && (q & 1u))) ++q;
-    bits = q;  // may carry into the exponent field: that is the correct rounding
-  } else {
-    uint32_t q = mant >> 13;
-    const uint32_t rem = mant & 0x1fffu;
-    if (rem > 0x1000u || (rem == 0x1000u && (q & 1u))) ++q;
-    // q in [0x400, 0x800]; exponent field e+15, carry handled by the addition
-    bits = (static_cast<uint32_t>(e + 15) << 10) + (q - 0x400u);
-    if (bits >= 0x7c00u) bits = 0x7c00u;  // overflow to inf
-  }
-  return static_cast<uint16_t>(sign | bits);
+  // Subnormal half: value = mant * 2^(e-23); half ulp is 2^-24.
+  const int shift = -e - 14 + 13;  // 14..24
+  uint32_t q = mant >> shift;
+  const uint32_t rem = mant & ((1u << shift) - 1u);
+  const uint32_t halfway = 1u << (shift - 1);
+  if (rem > halfway || (rem == halfway && (q & 1u))) ++q;
+  return static_cast<uint16_t>(sign | q);  // may carry into the exponent field: that is the correct rounding
 }
 
 // fp32 -> fp16 as the reference's load-time model converter rounds
