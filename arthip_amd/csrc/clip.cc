@@ -359,6 +359,11 @@ bool ClipModel::GetFrame(const VideoFormat& fmt, const int* plane_w, const int* 
   for (int c = 0; c < need; ++c)
     if (dst[c] == nullptr) return fail("null destination plane");
 
+  struct InFlight {
+    std::atomic<int>& n;
+    explicit InFlight(std::atomic<int>& c) : n(c) { ++n; }
+    ~InFlight() { --n; }
+  } in_flight(in_flight_);
   std::unique_lock<std::mutex> lock;
   Io* io = nullptr;
   Slot& s = Acquire(lock, io);
@@ -497,9 +502,15 @@ bool ClipModel::RunSlot(Slot& s, Io& io, const VideoFormat& fmt, int in_c, int w
         (int_out && !grow_dev(io.out_int_dev, io.out_int_cap, dl_bytes, aerr)))
       return fail(aerr);
     // Small transfers are kernels on the engine's own stream, without the copy
-    // streams and their events.
+    // streams and their events. With other frames in flight, larger uploads
+    // overlap their kernels on the copy stream instead: a frame of the shipped
+    // architecture in a queue of two at 480x853 GRAY8 (0.41 MB) 757 -> 753 us, at
+    // 720p (0.92 MB) 1515 -> 1502, but C4F32 at 270x480 (0.13 MB) 68 -> 84.
+    // Alone, 720p takes 1787 us against 1796. Downloads up to the limit are
+    // faster by kernel in either case (C4F32 at 270x480, 1.04 MB, in that 68).
     void* upload_dst = direct_in ? io.in_dev : io.raw_dev;
-    if (raw_bytes <= kKernelCopyBytes) {
+    const size_t kernel_upload = in_flight_.load() > 1 ? kSharedKernelUploadBytes : kKernelCopyBytes;
+    if (raw_bytes <= kernel_upload) {
       if ((e = launch_copy(upload_dst, io.raw_host, raw_bytes, s.stream)) != hipSuccess)
         return drain(hip_fail("HIP input upload", e));
     } else if ((e = hipMemcpyAsync(upload_dst, io.raw_host, raw_bytes, hipMemcpyHostToDevice, s.up)) != hipSuccess ||

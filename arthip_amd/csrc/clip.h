@@ -106,6 +106,7 @@ class ClipModel {
   std::unique_ptr<CopyStreams> copy_;
   std::vector<std::unique_ptr<Slot>> slots_;
   std::atomic<unsigned> next_{0};
+  std::atomic<int> in_flight_{0};  // frames inside GetFrame
   // VSHIP_PROFILE=1 at creation: per-launch GPU spans and the output
   // conversion + download span on stderr for the first three frames of each
   // engine and every 128th (hip_engine.cc:1409-1604).

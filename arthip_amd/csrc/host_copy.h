@@ -15,6 +15,8 @@ namespace arthip {
 // stream and the kernels cost more than the bytes (R8F64 at 64x96 host to host
 // 114 -> 110 us, a 270x480 frame through the filter 306 -> 288 us).
 constexpr size_t kKernelCopyBytes = static_cast<size_t>(1) << 20;
+// The filter's limit for uploads while other frames are in flight.
+constexpr size_t kSharedKernelUploadBytes = static_cast<size_t>(256) << 10;
 
 // `rows` rows of `row` bytes, `stride` bytes apart, of the caller's memory.
 struct HostRows {

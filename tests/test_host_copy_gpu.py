@@ -44,3 +44,20 @@ def test_filter_rows(h, w):
         for pad in (0, 5):
             (y,) = m.get_frame([x[0, 0]], out_row_pad=pad)
             np.testing.assert_array_equal(y.view(np.uint16), want.view(np.uint16))
+
+
+# Uploads of 2 h w bytes with several callers: below 256 KiB always by kernel;
+# up to 1 MiB by kernel or on the copy stream, as other frames are in flight or not;
+# above on the copy stream.
+@pytest.mark.parametrize("h,w", [(250, 511), (256, 513), (480, 853), (733, 1011)])
+def test_filter_with_several_callers(h, w):
+    from concurrent.futures import ThreadPoolExecutor
+    spec = models.c4f32(seed=1)
+    xs = [models.synthetic_input((1, 1, h, w), seed=s) for s in range(5)]
+    with Engine(0) as e:
+        e.build(spec)
+        want = [_device_run(e, x)[0, 0].view(np.uint16) for x in xs]
+    with vs.Model("GRAYH", w, h, spec.bytes()) as m, ThreadPoolExecutor(4) as pool:
+        got = list(pool.map(lambda i: m.get_frame([xs[i % 5][0, 0]])[0].view(np.uint16), range(40)))
+    for i, y in enumerate(got):
+        np.testing.assert_array_equal(y, want[i % 5])
