@@ -419,16 +419,29 @@ def launch_work(spec, steps, px: int):
             ci += 1
             b = 2.0 * px * (c + m * (1 + nsk)) + 18.0 * c * m
             fd = 2.0 * 9 * px * c * m
-            # The row pipes run the fused block's row scheme (6/9 of direct): a
-            # lone 64 -> 64 conv without residual inputs, a 96 -> 96 conv with
-            # at most one. Other convs F(2x2,3x3) (16/36).
-            rows = (c == m == 64 and nsk == 0) or (c == m == 96 and nsk <= 1)
-            direct = c == 1 or 16 <= c <= 48  # direct.hip at the body widths
-            fw = fd if direct else fd * 6 / 9 if rows else fd * 16 / 36
+            fw = fd * products_share(c, m, nsk, last=ci == len(convs))
             out.append({"bytes": b, "flops_direct": fd, "flops_wino": fw, "convs": 1})
         else:
             out.append(None)
     return out
+
+
+def products_share(c: int, m: int, nsk: int, last: bool) -> float:
+    """Products that the kernel of a conv launched alone executes, as a share of
+    the direct conv's (launch_winograd's choice at 16-byte aligned buffers)."""
+    if c == 1:
+        return 1.0  # the one-channel head
+    if last and m <= 16:  # boundary outputs
+        return 1.0 if c in (32, 64, 96) and nsk == 0 else 16 / 36
+    if 2 <= c <= 4 and m in (32, 64, 96) and nsk == 0:
+        return 1.0  # conv3x3_head
+    if c % 8 == 0 and 16 <= c <= 48 and m % 8 == 0 and 8 <= m <= 48:
+        return 1.0  # conv3x3_rows
+    # The row pipes run the fused block's row scheme: a lone 64 -> 64 conv without
+    # residual inputs, a 96 -> 96 conv with at most one.
+    if (c == m == 64 and nsk == 0) or (c == m == 96 and nsk <= 1):
+        return 6 / 9
+    return 16 / 36  # F(2x2,3x3)
 
 
 def frame_bytes(spec, work, n, h, w, oshape, roofline) -> dict:

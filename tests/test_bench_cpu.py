@@ -52,6 +52,20 @@ def test_launch_work_counts_each_distinct_tensor_once():
     assert got[1] == 2 * act + 18.0 * 64 * 64
 
 
+def test_products_share_follows_the_dispatch():
+    """Direct kernels: heads of one to four channels, body widths 16 to 48 in
+    multiples of eight, narrow boundary outputs. Row Winograd: lone 64 -> 64, 96 ->
+    96 with at most one residual. Everything else F(2x2,3x3)."""
+    share = bench.products_share
+    for c, m, nsk in ((1, 64, 0), (2, 32, 0), (3, 64, 0), (4, 96, 0), (16, 8, 0), (32, 32, 2), (40, 48, 1)):
+        assert share(c, m, nsk, False) == 1.0, (c, m, nsk)
+    for c, m, nsk in ((3, 64, 1), (3, 48, 0), (5, 64, 0), (20, 32, 0), (32, 64, 0), (48, 12, 0), (64, 64, 1),
+                      (96, 96, 2)):
+        assert share(c, m, nsk, False) == 16 / 36, (c, m, nsk)
+    assert share(64, 64, 0, False) == share(96, 96, 1, False) == 6 / 9
+    assert share(64, 4, 0, True) == 1.0 and share(16, 16, 0, True) == 16 / 36
+
+
 def test_end_to_end_reports_a_failed_filter_child(monkeypatch):
     """The VapourSynth-path rate runs in a child process; if the child fails,
     the bench line carries null and the error instead of failing as a whole."""
