@@ -1,6 +1,8 @@
-// Direct 3x3 convs on the matrix cores for narrow layers (padded NHWC fp16 in
-// and out): the head of a model with two to four input channels
-// (conv3x3_head).
+// Direct 3x3 convs on the matrix cores for narrow layers, padded NHWC fp16 in
+// and out: the head of a model with two to four input channels (conv3x3_head)
+// and body convs of 16 to 48 channels (conv3x3_rows). For the 32-channel model,
+// two convs in one launch at either boundary: the one-channel head and the conv
+// after it (conv3x3_head_pair), the last conv and the tail (conv3x3_tail_pair).
 
 #include <hip/hip_runtime.h>
 
@@ -23,9 +25,11 @@ constexpr uint32_t kOob = 0x80000000u;
 // In NHWC the three pixels of a kernel row are 3 C contiguous values, so one
 // v_mfma_f32_16x16x32_f16 takes the first eight values of all three rows: lane
 // (q, j) supplies row q of pixel j (q = 3: zeros). Values 8 .. 11 (C = 3, 4) go
-// to a second one laid out the same way (a K = 16 product would hold them, but
-// v_mfma_f32_16x16x16_f16 accumulating onto a K = 32 result gave wrong values in
-// the result's first two registers). A holds the taps in the same slots (packed
+// to a second one laid out the same way. (A K = 16 product would hold them, but
+// hipcc issues a v_mfma_f32_16x16x16_f16 that adds to a K = 32 result right behind
+// it, without wait states, as it does for products of one shape; the first two
+// registers of the sum were then wrong, as if read before they were written. No
+// kernel adds one shape onto another.) A holds the taps in the same slots (packed
 // by winograd_pack, zero where no tap is), its channels permuted so that lane
 // (q, j) ends with the contiguous channels 4 NB q .. 4 NB q + 4 NB - 1 of pixel j.
 //

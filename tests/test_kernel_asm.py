@@ -121,3 +121,50 @@ def test_drain_check_catches_a_missing_drain():
     assert _drained(["ds_write_b128 v1, v[2:5]", "s_waitcnt lgkmcnt(0)", "v_add_u32 v1, v2, v3",
                      "s_barrier"], 3)
     assert not _drained([":label", "v_add_u32 v1, v2, v3", "s_barrier"], 2)
+
+
+def _regs(operand):
+    m = re.fullmatch(r"([va])(?:\[(\d+):(\d+)\]|(\d+))", operand.strip())
+    if not m:
+        return set()
+    lo = int(m.group(2) or m.group(4))
+    return {(m.group(1), r) for r in range(lo, int(m.group(3) or lo) + 1)}
+
+
+def _mixed_accumulators(ins):
+    """Matrix products that accumulate onto the result of one of another shape in
+    their basic block."""
+    shape = {}  # register -> shape of the product that wrote it last
+    bad = []
+    for t in ins:
+        if t == ":label":
+            shape.clear()
+            continue
+        op, _, rest = t.partition(" ")
+        args = [a for a in re.split(r",\s*(?![^\[]*\])", rest.strip())]
+        mfma = re.match(r"v_mfma_\w+?_(\d+x\d+x\d+)", op)
+        if mfma and any(shape.get(r, mfma.group(1)) != mfma.group(1) for r in _regs(args[3].split()[0])):
+            bad.append(t)
+        for r in _regs(args[0].split()[0] if args[0] else ""):
+            if mfma:
+                shape[r] = mfma.group(1)
+            elif not op.startswith(("ds_write", "global_store", "buffer_store")):
+                shape.pop(r, None)
+    return bad
+
+
+def test_no_product_accumulates_onto_another_shape(kernel_asm):
+    """hipcc issues v_mfma_f32_16x16x16_f16 right behind the v_mfma_f32_16x16x32_f16
+    whose result it adds to, with no wait states, as it does for products of one
+    shape; on the GPU the first two registers of the sum were wrong then. No kernel
+    may hold such a pair."""
+    products = 0
+    for name, ins in _kernels(kernel_asm):
+        products += sum(t.startswith("v_mfma") for t in ins)
+        assert not _mixed_accumulators(ins), (name, _mixed_accumulators(ins)[:3])
+    assert products > 1000
+    first = "v_mfma_f32_16x16x32_f16 v[0:3], v[2:5], v[10:13], v[6:9]"
+    assert _mixed_accumulators([first, "v_mfma_f32_16x16x16_f16 v[0:3], v[14:15], v[4:5], v[0:3]"])
+    assert not _mixed_accumulators([first, "v_mfma_f32_16x16x32_f16 v[0:3], v[2:5], v[4:7], v[0:3]"])
+    assert not _mixed_accumulators([first, "v_add_f32_e32 v0, v0, v8", "v_add_f32_e32 v1, v1, v8", "v_mov_b32_e32 v2, 0",
+                                    "v_mov_b32_e32 v3, 0", "v_mfma_f32_16x16x16_f16 v[0:3], v[4:5], v[4:5], v[0:3]"])
