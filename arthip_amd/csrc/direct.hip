@@ -207,11 +207,13 @@ __global__ void __launch_bounds__(256) conv3x3_head(DirectRowArgs a) {
 // ring pixel p at g ^ (2 ((p >> 2) & 1)) (on the copies' source side), which is
 // too; C = 24 and 40 read two-way.
 //
-// The stream through memory bounds it, on small images the launch and the first
-// rows' latency. 48 -> 48 + ReLU at 541x963 (100 MB): 61 us in winograd_conv, 29
-// here; 32 -> 32 + ReLU at 540x960 (66 MB): 24 us in the strip kernel it ran on
-// before, 17 here; with a residual at 1080p (398 MB): 88 and 65 us; 16 -> 16 at
-// 1080p (133 MB): 68 and 26 us. Its error against 64 bits is a third of
+// The stream through memory bounds it at full frames (32 -> 32 with a residual at
+// 1080p, 398 MB: 88 us in the strip kernel it ran on before, 63 here, 6.5 TB/s).
+// On nine-row runs nothing does alone (48 -> 48 + ReLU at 541x963, 100 MB: 65 us
+// in winograd_conv, 30 here; 3.8 TB/s, matrix units 32% busy, LDS 21%): each
+// run's first rows and a wave's own chain a step, two waves per SIMD. 32 -> 32 +
+// ReLU at 540x960 (66 MB): 24 and 17 us; 16 -> 16 at 1080p (133 MB): 68 and 26.
+// (Kernel times; whole calls take about 1 us more.) Its error against 64 bits is a third of
 // Winograd's (2.1e-4 against 6.1e-4): no transform rounds its inputs.
 template <int C, int OB, int NSKIP>
 struct RowsL {
@@ -469,9 +471,11 @@ conv3x3_rows(DirectRowArgs a) {
 // output tensor never exists. Step k computes head row k + 3 while it folds rows
 // k .. k + 2; the input of the row after that is requested a step ahead. Head
 // pixels outside the image are zero: the second conv's padding.
-// The output's write stream and the launch bound it. At 540x960: 11 us for the
-// head and 17 for the conv apart, 20 here; the 32-channel model's frame 62.7 -> 54.7
-// us, at 2x1080x1920 390 -> 301.
+// No unit is the bound at 540x960 (matrix units 18% busy, LDS 20%, 1.6 TB/s
+// written): the launch, and a wave's own chain a step (input, head product, LDS,
+// nine folds, staging, stores) with two waves per SIMD over nine rows. Head and
+// conv apart 11 + 17 us there, 21 here; the 32-channel model's frame 62.7 -> 54.7 us
+// (with the tail still apart), at 2x1080x1920 390 -> 301.
 struct HeadPairL : RowsL<32, 2, 0> {
   static constexpr int R = 4;
   static constexpr int STG = R * SLOT;
@@ -675,8 +679,9 @@ conv3x3_head_pair(HeadPairArgs a) {
 // q < 2, ends with the two values of output row 2 y + q at pixel 2 x: one store
 // per tile, bias, activation and Clip in fp32 before it.
 // Every step issues NI copies (LA rows ahead) and NST stores.
-// The LDS reads and writes of a step, and at small sizes the launch and the fill of
-// a run, bound it. The 32-channel model's frame with conv and tail apart and in
+// At 540x960 a run is 14 steps for nine rows, and no unit is the bound (25 us;
+// matrix units 34% busy, LDS 12%, 2 TB/s): the launch and a wave's own chain a step,
+// two waves per SIMD. The 32-channel model's frame with conv and tail apart and in
 // one launch: 54.3 -> 47.2 us at 540x960, 155.7 -> 121 at 1080p, 300 -> 220 at
 // 2x1080x1920.
 struct TailPairL : RowsL<32, 2, 0> {

@@ -12,8 +12,9 @@ namespace arthip {
 
 // Transfers up to this size go by a copy kernel on the launch stream between
 // pinned and device memory: a copy engine's start and the waits between its
-// stream and the kernels cost more than the bytes (R8F64 at 64x96 host to host
-// 114 -> 110 us, a 270x480 frame through the filter 306 -> 288 us).
+// stream and the kernels cost more than the bytes (through the filter, copy
+// streams and kernels with everything else alike: C4F32 at 96x128 85 -> 51 us a
+// frame, at 270x480 140 -> 119, the shipped architecture at 270x480 454 -> 424).
 constexpr size_t kKernelCopyBytes = static_cast<size_t>(1) << 20;
 // The filter's limit for uploads while other frames are in flight.
 constexpr size_t kSharedKernelUploadBytes = static_cast<size_t>(256) << 10;
@@ -31,9 +32,12 @@ struct HostRows {
 // travel. The copy out of memory that the GPU has just written runs at about
 // half the link's rate on one thread, and the first write to a fresh
 // destination page faults, so larger frames are shared with up to three helper
-// threads, which touch the destination while the GPU still works; they end with
-// the call. Through the filter, C4F32 at 1080p (16.6 MB out) 1460 -> 980 us, the
-// shipped architecture at 720p (7.4 MB out) 2060 -> 1880 us.
+// threads, which touch the destination and then sleep while the GPU still works;
+// they end with the call. Through the filter, one chunk on the caller's thread
+// against this: one caller, C4F32 at 1080p (16.6 MB out) 1130 -> 790 us a frame,
+// R8F64 there 2700 -> 2370, the shipped architecture at 720p (7.4 MB out) 1830 ->
+// 1720; two callers, C4F32 610 -> 425, R8F64 the same (1790). CPU time a frame
+// grows by the helpers: R8F64 3.0 -> 3.7 ms, with two callers 3.9 -> 4.9.
 class ChunkedDownload {
  public:
   ChunkedDownload() = default;
