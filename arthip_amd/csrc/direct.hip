@@ -215,16 +215,19 @@ __global__ void __launch_bounds__(256) conv3x3_head(DirectRowArgs a) {
 // ReLU at 540x960 (66 MB): 24 and 17 us; 16 -> 16 at 1080p (133 MB): 68 and 26.
 // (Kernel times; whole calls take about 1 us more.) Its error against 64 bits is a third of
 // Winograd's (2.1e-4 against 6.1e-4): no transform rounds its inputs.
-template <int C, int OB, int NSKIP>
+//
+// C = 24 and 40 take four tiles a step, whose ring rows are whole copies, and two
+// (rows_two_tiles) where that is slower than winograd_conv was.
+template <int C, int OB, int NSKIP, int TILES = C % 16 == 0 ? 2 : 4>
 struct RowsL {
-  // 16-pixel tiles per step; four where two tiles' row is not whole copies.
-  static constexpr int T = C % 16 == 0 ? 2 : 4;
+  static constexpr int T = TILES;        // 16-pixel tiles per step
   static constexpr int IPX = 16 * T;     // input pixels per ring row
   static constexpr int OPX = IPX - 2;    // output pixels per segment, at most
   static constexpr int PXB = 2 * C;      // input bytes per pixel
   static constexpr int KR = (3 * C + 31) / 32;
   static constexpr int VO = 3 * C / 8 - 4 * (KR - 1);  // octets of the last product
-  static constexpr int NI = IPX * PXB / 1024;          // copies per row
+  // Copies per row (C = 24 and 40 with two tiles: half of the last out of range).
+  static constexpr int NI = (IPX * PXB + 1023) / 1024;
   static constexpr int SLOT = NI * 1024;
   static constexpr int LA = 2;
   static constexpr int R = LA + 3;
@@ -234,10 +237,9 @@ struct RowsL {
   static constexpr int STG = R * SLOT;
   // Reads of the last tile's unused columns run past the last slot.
   static constexpr size_t lds_bytes() { return STG + (NSKIP == 0 ? 1 : 2 * NSKIP) * SSLOT; }
-  static_assert(IPX * PXB % 1024 == 0, "whole copies");
   static_assert((LA - 1) * (NI + NSK) + LA * NS < 64 && 2 * NI + NS + NSK < 64, "vmcnt field");
   static_assert(NS <= (LA + 1) * NI, "the first residual row's wait");
-  // Last byte read in a slot: pixel 63's row of KR products.
+  // Last byte read in a slot: the last pixel's row of KR products.
   static_assert((IPX - 1) * PXB + 64 * KR - SLOT <= SSLOT, "reads stay inside the LDS");
 };
 
@@ -298,11 +300,11 @@ __device__ __forceinline__ void rows_store(const char* lin, __amdgpu_buffer_rsrc
                                            (uint32_t)(1024 * i + 16 * lane), 0, AUX);
 }
 
-template <int C, int OB, int NSKIP>
+template <int C, int OB, int NSKIP, int TILES>
 __global__ void __launch_bounds__(64)
     __attribute__((amdgpu_waves_per_eu(2)))
 conv3x3_rows(DirectRowArgs a) {
-  using L = RowsL<C, OB, NSKIP>;
+  using L = RowsL<C, OB, NSKIP, TILES>;
   constexpr int T = L::T, KR = L::KR, NI = L::NI, NS = L::NS, NSK = L::NSK, LA = L::LA, R = L::R;
   constexpr bool SWZ = C == 32;
   extern __shared__ __attribute__((aligned(16))) char rlds[];
@@ -897,20 +899,48 @@ RowKernel head_kernel(int M, int act) {
                                                         : head_kernel_act<C, 6>(act);
 }
 
+// Two tiles a step at C = 24 and 40, for more than 32 outputs: without a residual
+// input at C = 40, where the taps and sums of four spill (40 -> 40 at 361x481 16.9
+// against 11.6 us, 1080p 115 and 73; winograd_conv 24 and 259), and on up to 2^15
+// pixels, where a launch is one short run a wave and four tiles make it longer
+// (24 -> 40 + two residuals at 16x16 4.6 and 3.6 us, 100x160 5.0 and 4.2, 300x64 5.4
+// and 4.5; winograd_conv 4.0, 4.3, 4.9). Above, four are up to 17% faster on runs of
+// one row (200x300: 6.3 and 7.4).
+constexpr bool rows_two_tiles(int C, int M, int nskip, int64_t pixels) {
+  return C % 16 != 0 && M > 32 && (pixels <= 1 << 15 || (C == 40 && nskip == 0));
+}
+
+struct RowsPick {
+  RowKernel fn = nullptr;
+  size_t lds = 0;
+  int seg = 0;  // output pixels per segment, at most
+};
+
+template <int C, int OB, int NSKIP>
+RowsPick rows_pick(bool two) {
+  auto of = [](auto tiles) {
+    using L = RowsL<C, OB, NSKIP, decltype(tiles)::value>;
+    return RowsPick{conv3x3_rows<C, OB, NSKIP, decltype(tiles)::value>, L::lds_bytes(), L::OPX};
+  };
+  if constexpr (C % 16 == 0 || rows_two_tiles(C, 16 * OB, NSKIP, (int64_t)1 << 40))
+    return of(IntC<2>{});
+  else if constexpr (!rows_two_tiles(C, 16 * OB, NSKIP, 1))
+    return of(IntC<4>{});
+  else
+    return two ? of(IntC<2>{}) : of(IntC<4>{});
+}
+
 template <int C, int OB>
-RowKernel rows_kernel(int nskip, size_t* lds) {
-  switch (nskip) {
-    case 0: *lds = RowsL<C, OB, 0>::lds_bytes(); return conv3x3_rows<C, OB, 0>;
-    case 1: *lds = RowsL<C, OB, 1>::lds_bytes(); return conv3x3_rows<C, OB, 1>;
-    default: *lds = RowsL<C, OB, 2>::lds_bytes(); return conv3x3_rows<C, OB, 2>;
-  }
+RowsPick rows_pick(int nskip, bool two) {
+  return nskip == 0 ? rows_pick<C, OB, 0>(two) : nskip == 1 ? rows_pick<C, OB, 1>(two) : rows_pick<C, OB, 2>(two);
 }
 
 template <int C>
-RowKernel rows_kernel(int M, int nskip, size_t* lds) {
-  return M <= 16   ? rows_kernel<C, 1>(nskip, lds)
-         : M <= 32 ? rows_kernel<C, 2>(nskip, lds)
-                   : rows_kernel<C, 3>(nskip, lds);
+RowsPick rows_pick(int M, int nskip, int64_t pixels) {
+  const bool two = rows_two_tiles(C, M, nskip, pixels);
+  return M <= 16   ? rows_pick<C, 1>(nskip, two)
+         : M <= 32 ? rows_pick<C, 2>(nskip, two)
+                   : rows_pick<C, 3>(nskip, two);
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -1004,38 +1034,35 @@ hipError_t launch_conv_head(const WinoArgs& w, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Output pixels of a conv3x3_rows segment.
-static int rows_segment(int C) { return C % 16 == 0 ? RowsL<16, 1, 0>::OPX : RowsL<24, 1, 0>::OPX; }
-
 bool conv_rows_eligible(const WinoArgs& w) {
   const int64_t cm = w.C > w.M ? w.C : w.M;
   return inner_epilogue(w) && direct_rows_shape(w.C, w.M) && aligned16(w.in) &&
          aligned16(w.epi.out) && aligned16(w.epi.skip0) && aligned16(w.epi.skip1) &&
-         fits32(w.N, w.H, w.W, cm, rows_segment(w.C));
+         fits32(w.N, w.H, w.W, cm, RowsL<16, 1, 0>::OPX);  // (the shorter segment)
 }
 
 hipError_t launch_conv_rows(const WinoArgs& w, hipStream_t s) {
   if (!conv_rows_eligible(w)) return hipErrorInvalidValue;
-  DirectRowArgs a = row_args(w, rows_segment(w.C));
-  a.nt_out = nt_stores(a);
-  const int nskip = (a.skip0 != nullptr) + (a.skip1 != nullptr);
-  size_t lds = 0;
-  RowKernel fn = nullptr;
+  const int nskip = (w.epi.skip0 != nullptr) + (w.epi.skip1 != nullptr);
+  const int64_t pixels = (int64_t)w.N * w.H * w.W;
+  RowsPick k;
   switch (w.C) {
-    case 16: fn = rows_kernel<16>(w.M, nskip, &lds); break;
-    case 24: fn = rows_kernel<24>(w.M, nskip, &lds); break;
-    case 32: fn = rows_kernel<32>(w.M, nskip, &lds); break;
-    case 40: fn = rows_kernel<40>(w.M, nskip, &lds); break;
-    case 48: fn = rows_kernel<48>(w.M, nskip, &lds); break;
+    case 16: k = rows_pick<16>(w.M, nskip, pixels); break;
+    case 24: k = rows_pick<24>(w.M, nskip, pixels); break;
+    case 32: k = rows_pick<32>(w.M, nskip, pixels); break;
+    case 40: k = rows_pick<40>(w.M, nskip, pixels); break;
+    case 48: k = rows_pick<48>(w.M, nskip, pixels); break;
     default: return hipErrorInvalidValue;
   }
+  DirectRowArgs a = row_args(w, k.seg);
+  a.nt_out = nt_stores(a);
   // Eight waves per CU at most: more make the runs shorter (two rows of halo
   // each) without streaming faster (32 -> 32 + residual at 1080p: 94 us with
   // twelve, 86 with eight, 84 with five; 16 -> 16 at 1080p: 24, 26, 36).
   unsigned blocks = 0;
-  const hipError_t e = rows_grid(fn, a, 64, lds, 8, 1, &blocks);
+  const hipError_t e = rows_grid(k.fn, a, 64, k.lds, 8, 1, &blocks);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(blocks), dim3(64), lds, s, a);
+  hipLaunchKernelGGL(k.fn, dim3(blocks), dim3(64), k.lds, s, a);
   return hipGetLastError();
 }
 

@@ -57,10 +57,11 @@ def test_head_nonfinite(c):
 
 
 # conv3x3_rows: one wave per segment of up to 30 pixels (C = 16, 32, 48: two
-# 16-pixel tiles) or 62 (C = 24, 40: four), one output row per step, input rows
-# two steps ahead: runs of one, two and three rows, one pixel less and more than a
-# tile and than a segment of either length, many rows per wave, several runs per
-# wave (many segments, few rows).
+# 16-pixel tiles) or 62 (C = 24, 40: four; but two for more than 32 outputs on up to
+# 2^15 pixels, and at C = 40 without a residual input on any), one output row per
+# step, input rows two steps ahead: runs of one, two and three rows, one pixel less
+# and more than a tile and than a segment of either length, many rows per wave,
+# several runs per wave (many segments, few rows).
 ROWS_SIZES = [(1, 1, 1), (2, 2, 15), (1, 3, 17), (1, 2, 29), (1, 4, 30), (2, 3, 31), (1, 5, 32), (3, 5, 61),
               (1, 2, 62), (1, 1, 63), (2, 4, 91), (2, 4, 125), (1, 700, 130), (1, 3, 4001), (2, 67, 1921)]
 
@@ -71,7 +72,8 @@ def _skips(seed, k, n, m, h, w):
 
 
 @pytest.mark.parametrize("n,h,w", ROWS_SIZES)
-@pytest.mark.parametrize("c,m,k", [(16, 16, 1), (24, 24, 2), (32, 32, 0), (48, 48, 1)])
+@pytest.mark.parametrize("c,m,k", [(16, 16, 1), (24, 24, 2), (32, 32, 0), (48, 48, 1), (24, 48, 2), (40, 40, 0),
+                                   (40, 40, 1)])
 def test_rows(c, m, k, n, h, w):
     x, wt, b = make_case(60, n, c, m, h, w)
     sk = _skips(61, k, n, m, h, w)
