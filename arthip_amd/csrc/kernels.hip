@@ -2661,7 +2661,10 @@ hipError_t launch_pipe(StripArgs a, int act, hipStream_t s) {
       }
   }
   grid = (grid + 7) / 8 * 8;
-  a.split = make_split(a.n_items, (int)grid, a.tiles_h, 3);
+  // Producers and consumers stream across strips without a drain, so entering
+  // one costs nothing and strips are not padded (96 -> 96 + two residuals with a
+  // fill of 3 items: 64x700 13.2 us against 12.1, 270x480 24.7 against 23.9).
+  a.split = make_split(a.n_items, (int)grid, a.tiles_h, 0);
   hipLaunchKernelGGL(pf, dim3((unsigned)grid), dim3(512), lds, s, a);
   return hipGetLastError();
 }
