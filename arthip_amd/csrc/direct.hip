@@ -213,11 +213,11 @@ __global__ void __launch_bounds__(256) conv3x3_head(DirectRowArgs a) {
 // in winograd_conv, 30 here; 3.8 TB/s, matrix units 32% busy, LDS 21%): each
 // run's first rows and a wave's own chain a step, two waves per SIMD. 32 -> 32 +
 // ReLU at 540x960 (66 MB): 24 and 17 us; 16 -> 16 at 1080p (133 MB): 68 and 26.
-// (Kernel times; whole calls take about 1 us more.) Its error against 64 bits is a third of
-// Winograd's (2.1e-4 against 6.1e-4): no transform rounds its inputs.
+// (Kernel times; whole calls take about 1 us more.) Its error against 64 bits is a
+// third of Winograd's (2.1e-4 against 6.1e-4): no transform rounds its inputs.
 //
 // C = 24 and 40 take four tiles a step, whose ring rows are whole copies, and two
-// (rows_two_tiles) where that is slower than winograd_conv was.
+// where those are the slower form (rows_two_tiles).
 template <int C, int OB, int NSKIP, int TILES = C % 16 == 0 ? 2 : 4>
 struct RowsL {
   static constexpr int T = TILES;        // 16-pixel tiles per step
